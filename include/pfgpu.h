@@ -95,7 +95,9 @@ typedef struct pfgpu_stats {
     int workgroups;       /* instance groups of G */
     int fallback_fp64;    /* FP32-form rows (or chains) re-solved in FP64 */
     /* wall clock of workgroup 0 per NR phase, summed over its iterations and instances:
-     * J fill, factor + forward solve, dense tail, backward solve, voltage update, mismatch */
+     * J fill, factor + forward solve, dense tail, backward solve, voltage update, mismatch. J and the
+     * mismatch's sums are assembled in one pass over Ybus, counted as J fill; its norm, the convergence
+     * test and the start of a solve count as mismatch (DC solves and re-pivoted plans: each by itself). */
     double phase_s[6];
     int block_size;           /* lanes per workgroup */
     int resident_workgroups;  /* workgroups launched (each loops over instance groups) */

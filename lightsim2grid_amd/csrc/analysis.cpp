@@ -379,6 +379,34 @@ namespace pfgpu {
 void recycle_slots(DevicePlan& P);
 void build_jfill_table(DevicePlan& P);
 
+void ybus_rows(const YbusPattern& Y, DevicePlan& P) {
+    const int n = Y.n, nnz = Y.p[n];
+    P.yr_ptr.assign(n + 1, 0);
+    for (int q = 0; q < nnz; ++q) P.yr_ptr[Y.i[q] + 1]++;
+    for (int r = 0; r < n; ++r) P.yr_ptr[r + 1] += P.yr_ptr[r];
+    P.yr_col.resize(nnz);
+    P.yr_pos.resize(nnz);
+    std::vector<int> f(P.yr_ptr.begin(), P.yr_ptr.end() - 1);
+    for (int c = 0; c < n; ++c)
+        for (int q = Y.p[c]; q < Y.p[c + 1]; ++q) {
+            const int k = f[Y.i[q]]++;
+            P.yr_col[k] = c;
+            P.yr_pos[k] = q;
+        }
+}
+
+FactorCounts factor_counts(const JPattern& J, const std::vector<int>& perm) {
+    const SymbolicLU S = symbolic_lu(J, 96, &perm);
+    FactorCounts c;
+    c.nnzLU = S.N + 2 * S.nnzL;
+    c.flops = S.flops;
+    for (int k = 0; k < S.k0; ++k) {
+        const int64_t a = S.cp[k + 1] - S.cp[k];
+        c.npairs += a * (a + 1);  // every entry of the arm's square, and its right-hand side
+    }
+    return c;
+}
+
 DevicePlan build_device_plan(const YbusPattern& Y, const JPattern& J, const SymbolicLU& S, const Schedule& sch) {
     DevicePlan P;
     const int n = Y.n, N = J.N;
@@ -436,20 +464,7 @@ DevicePlan build_device_plan(const YbusPattern& Y, const JPattern& J, const Symb
     P.nvals = tail_slots + (int)ord.size();
     auto ys = [&](int k) { return nw[S.off_y + k]; };  // slot of y/x for permuted index k
 
-    // --- Ybus row view ----------------------------------------------------
-    P.yr_ptr.assign(n + 1, 0);
-    for (int c = 0; c < n; ++c)
-        for (int q = Y.p[c]; q < Y.p[c + 1]; ++q) P.yr_ptr[Y.i[q] + 1]++;
-    for (int r = 0; r < n; ++r) P.yr_ptr[r + 1] += P.yr_ptr[r];
-    P.yr_col.resize(P.nnzY); P.yr_pos.resize(P.nnzY);
-    {
-        std::vector<int> f(P.yr_ptr.begin(), P.yr_ptr.end() - 1);
-        for (int c = 0; c < n; ++c)
-            for (int q = Y.p[c]; q < Y.p[c + 1]; ++q) {
-                const int k = f[Y.i[q]]++;
-                P.yr_col[k] = c; P.yr_pos[k] = q;
-            }
-    }
+    ybus_rows(Y, P);
     // --- F rows and unknowns --------------------------------------------
     const int npvpq = (int)J.pvpq.size(), npq = (int)J.pq.size(), off = J.off;
     // the F entry of J row r is the right-hand side of factored row row_of(r)

@@ -171,6 +171,17 @@ struct DevicePlan {
 
 DevicePlan build_device_plan(const YbusPattern& Y, const JPattern& J, const SymbolicLU& S, const Schedule& sch);
 
+// The Ybus row view of a plan (yr_ptr, yr_col, yr_pos).
+void ybus_rows(const YbusPattern& Y, DevicePlan& P);
+
+// Size of the scalar factorisation in the elimination order perm, as its plan reports it: factor
+// entries, multiply pairs outside the dense tail, flops of one refactorisation.
+struct FactorCounts {
+    int64_t nnzLU = 0, npairs = 0;
+    double flops = 0;
+};
+FactorCounts factor_counts(const JPattern& J, const std::vector<int>& perm);
+
 // Per-level team sizes (lanes per task, power of two, team * G <= 64) for a
 // launch with G interleaved instances and `nslot` lanes per instance.
 std::vector<int> level_teams(const std::vector<int>& lvl_ptr, const std::vector<int>& maxp, int G, int nslot);

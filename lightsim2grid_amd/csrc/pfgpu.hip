@@ -38,7 +38,10 @@
 
 #include "../../include/pfgpu.h"
 #include "analysis.hpp"
+#include "blocks.hpp"
 #include "engine.hpp"
+#include "nr_block.hpp"
+#include "nr_device.hpp"
 #include "wide.hpp"
 
 std::string& pfgpu_engine::last_error() {
@@ -83,13 +86,8 @@ using pfgpu_engine::guarded;
 
 constexpr int kMaxBlock = 1024;
 constexpr int kMaxGraphs = 8;  // captured launch sequences kept per grid
-constexpr int kMaxEdits = 8;  // Ybus edits per instance kept in LDS
 constexpr int kMaxWaves = kMaxBlock / 64;
 constexpr int kMaxG = 32;
-constexpr int kEll = 4;  // Ybus row entries read at a time in the mismatch (column groups of its table)
-typedef __attribute__((address_space(3))) double lds_dbl;
-typedef __attribute__((address_space(3))) int lds_int;
-typedef __attribute__((address_space(3))) unsigned char lds_u8;
 
 // Per-workgroup state of the NR kernel, in dynamic LDS after the value slots and the level
 // table. The kernel declares no static LDS, so its value slots start at LDS address 0.
@@ -99,10 +97,6 @@ __host__ __device__ constexpr int wg_state_bytes(int G, int NT) {
     return 8 * G * (NT / 64 + 2 + 2 * kMaxEdits) + 4 * (G * (7 + kMaxEdits) + 2);
 }
 
-// Per-row diagnostic flags written by the NR kernel (pfgpu_stats / the fallback passes):
-constexpr int kFlagStall = 1;   // not converged, but the last mismatch is below the stall level
-constexpr int kFlagGrowth = 2;  // a pivot lost more than the growth threshold to cancellation
-constexpr int kStatusNotRun = 8;  // chain step after the chain's first failure (NotInitError)
 // Host re-pivot threshold: a diagonal pivot is kept while it holds at least this fraction of its
 // column's largest candidate (klu_defaults' tol)
 constexpr double kRepivotTau = 1e-3;
@@ -114,8 +108,7 @@ struct KArgs {
     int n, N, nJ, nzero, nlev, nblev, nlds, nspill, single_slack, ninst, max_iter, m;
     double tol;
     const int *yr_ptr, *yr_col, *yr_pos, *fslot_p, *fslot_q, *ux_bus, *ux_slot;
-    const int2* yr_pc;     // per Ybus row entry: {CSC position, column bus}
-    const int2* yr_ell;    // [ell_w][n]: the entries of every row as in yr_pc, {-1, row} past its end
+    const int2* yr_ell;    // [ell_w][n]: {CSC position, column bus} of every row's entries, {-1, row} past its end
     // J fill by Ybus entry: position, {row bus, column bus}, 4 target slots, 4 J indices
     const int* ye_pos;
     const int2* ye_rc;
@@ -193,187 +186,6 @@ struct KArgs {
     // s_it counts half-steps, the reported iterations are P half-steps, max_iter bounds them.
     int fdpf;
 };
-
-struct c64 {
-    double re, im;
-};
-__device__ __forceinline__ c64 cmul(c64 a, c64 b) { return {a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re}; }
-__device__ __forceinline__ c64 cconj(c64 a) { return {a.re, -a.im}; }
-__device__ __forceinline__ c64 csub(c64 a, c64 b) { return {a.re - b.re, a.im - b.im}; }
-__device__ __forceinline__ c64 cadd(c64 a, c64 b) { return {a.re + b.re, a.im + b.im}; }
-__device__ __forceinline__ c64 ld_c(const double* p, int i) { return {p[2 * i], p[2 * i + 1]}; }
-
-// Reduce over the nslot lanes of one instance: shuffles inside the wave
-// (lanes g, g+G, ... of a wave), then the kWaves partials through LDS.
-template <int G, int NT, bool IS_MAX>
-__device__ __forceinline__ double inst_reduce(double v, lds_dbl* part) {
-    constexpr int kWaves = NT / 64;
-#pragma unroll
-    for (int o = G; o < 64; o <<= 1) {
-        const double u = __shfl_xor(v, o);
-        v = IS_MAX ? fmax(v, u) : fmin(v, u);
-    }
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    __syncthreads();
-    if (lane < G) part[wave * G + lane] = v;
-    __syncthreads();
-    const int g = threadIdx.x % G;
-    double r = part[g];
-#pragma unroll
-    for (int k = 1; k < kWaves; ++k) r = IS_MAX ? fmax(r, part[k * G + g]) : fmin(r, part[k * G + g]);
-    return r;
-}
-
-// J value at the current V / Ibus (dS_dVa / dS_dVm, BaseNRAlgo.tpp:202-260) of a J entry
-// with selector sel (0/1: Re/Im dS_dVa, 2/3: Re/Im dS_dVm, 4: constant cv) built on the
-// Ybus entry y = Y(r, c); diag says r == c.
-__device__ __forceinline__ double jvalue_of(int sel, bool diag, c64 y, c64 vr, c64 vc, c64 ib, double cv) {
-    if (sel == 4) return cv;
-    if (sel >= 2) {
-        const double ic = 1.0 / sqrt(vc.re * vc.re + vc.im * vc.im);
-        c64 d = cmul(cconj(cmul(y, {vc.re * ic, vc.im * ic})), vr);
-        if (diag) {
-            const double ir = 1.0 / sqrt(vr.re * vr.re + vr.im * vr.im);
-            d = cadd(d, cmul(cconj(ib), {vr.re * ir, vr.im * ir}));
-        }
-        return sel == 2 ? d.re : d.im;
-    }
-    c64 t = cmul(y, vc);
-    if (diag) t = csub(t, ib);
-    const c64 d = cmul(cconj({-t.re, -t.im}), {-vr.im, vr.re});  // * (j V_r)
-    return sel == 0 ? d.re : d.im;
-}
-
-// Orders LDS accesses between the lanes of one wave (they run in lockstep; the
-// fence makes the compiler wait for outstanding LDS operations and not reorder).
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-    __builtin_amdgcn_wave_barrier();
-}
-
-__device__ __forceinline__ double inf_if_nonfinite(double a) { return (a <= 1.7976931348623157e308) ? a : INFINITY; }
-
-// Polar <-> rectangular conversions of one lane's buses (b0, b0 + step, ...).
-// Kept out of line: inlined FP64 atan2 / sincos raise the NR kernel's register
-// count past 128 VGPRs, which at 1024 lanes per workgroup means scratch spills
-// in the factor loop.
-// Va = arg(V), Vm = |V| (BaseNRAlgo.tpp:77-79, BaseNRSingleSlackAlgo.tpp:131-132)
-// V holds bus b at V[2 b vs] (vs = 1 in global memory, G in LDS).
-template <typename VP>
-__device__ __noinline__ void polar_of(VP V, int vs, double* __restrict__ Va, double* __restrict__ Vm, int b0, int n,
-                                      int step) {
-    for (int b = b0; b < n; b += step) {
-        const double vr = V[2 * b * vs], vi = V[2 * b * vs + 1];
-        Va[b] = atan2(vi, vr);
-        Vm[b] = sqrt(vr * vr + vi * vi);
-    }
-}
-// V = Vm * exp(j Va) (BaseNRAlgo.tpp:150-151); returns min Vm over the lane's buses
-template <typename VP>
-__device__ __noinline__ double rect_of(VP V, int vs, const double* __restrict__ Va, const double* __restrict__ Vm,
-                                       int b0, int n, int step) {
-    double vmin = INFINITY;
-    for (int b = b0; b < n; b += step) {
-        double sn, cs;
-        sincos(Va[b], &sn, &cs);
-        const double m = Vm[b];
-        V[2 * b * vs] = m * cs;
-        V[2 * b * vs + 1] = m * sn;
-        vmin = fmin(vmin, m);
-    }
-    return vmin;
-}
-
-// One bus of the voltage update (BaseNRAlgo.tpp:138-151): Va and Vm (taken from V first in
-// the single-slack form, BaseNRSingleSlackAlgo.tpp:131-132) minus the Newton step, then
-// V = Vm exp(j Va); returns Vm.
-template <typename VP>
-__device__ __noinline__ double update_bus(VP V, int vs, double* __restrict__ Va, double* __restrict__ Vm, int b,
-                                          double dva, double dvm, bool polar_first) {
-    double va, vm;
-    if (polar_first) {
-        const double vr = V[2 * b * vs], vi = V[2 * b * vs + 1];
-        va = atan2(vi, vr);
-        vm = sqrt(vr * vr + vi * vi);
-    } else {
-        va = Va[b];
-        vm = Vm[b];
-    }
-    va -= dva;
-    vm -= dvm;
-    Va[b] = va;
-    Vm[b] = vm;
-    double sn, cs;
-    sincos(va, &sn, &cs);
-    V[2 * b * vs] = vm * cs;
-    V[2 * b * vs + 1] = vm * sn;
-    return vm;
-}
-
-// Lane streams. Level l uses lanes [0, U) with K items per lane, item k of lane s
-// at base + k * U + s. End word (forward: item.w, backward: item.z): bits 0-24
-// slot, 25 assign (a fill-in entry: its slot held another value before), 26-28
-// log2(team), 29 reciprocal, 30 end of task, 31 the lane's last item of the level
-// (the lane loads nothing after it).
-constexpr int kSC = 2;  // items per prefetch group of the general walk
-constexpr int kHB = 4;  // items of a level loaded ahead, during the level before it (lean walk)
-constexpr int kEnd = 1 << 30;
-__device__ __forceinline__ int4 no_item() { return int4{-1, -1, 0, 0}; }
-
-// Moves v from lane + D to each lane (D < 16: within a row of 16 lanes by DPP row_shl,
-// no LDS traffic; lanes whose source is outside the row get 0).
-template <int D>
-__device__ __forceinline__ float lane_down(float v) {
-    if constexpr (D < 16) {
-        return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x100 + D, 0xF, 0xF, true));
-    } else {
-        return __shfl_down(v, D);
-    }
-}
-template <int D>
-__device__ __forceinline__ double lane_down(double v) {
-    if constexpr (D < 16) {
-        const long long b = __builtin_bit_cast(long long, v);
-        const int lo = __builtin_amdgcn_update_dpp(0, (int)(b & 0xffffffffLL), 0x100 + D, 0xF, 0xF, true);
-        const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0x100 + D, 0xF, 0xF, true);
-        return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned int)lo);
-    } else {
-        return __shfl_down(v, D);
-    }
-}
-
-// Sum over a team of 2^lt lanes (stride G, aligned to 2^lt * G) into its lowest lane.
-// maxlt (uniform) bounds the steps; lanes of smaller teams drop the later steps by a
-// select, not a branch. All lanes of a team share lt, so the lanes a leader reads are
-// active and in its team.
-template <int G, typename FT>
-__device__ __forceinline__ FT team_sum(FT acc, int lt, int maxlt) {
-    if (maxlt > 0) { const FT t = lane_down<1 * G>(acc); acc += lt > 0 ? t : (FT)0; }
-    if constexpr (2 * G <= 32) if (maxlt > 1) { const FT t = lane_down<2 * G>(acc); acc += lt > 1 ? t : (FT)0; }
-    if constexpr (4 * G <= 32) if (maxlt > 2) { const FT t = lane_down<4 * G>(acc); acc += lt > 2 ? t : (FT)0; }
-    if constexpr (8 * G <= 32) if (maxlt > 3) { const FT t = lane_down<8 * G>(acc); acc += lt > 3 ? t : (FT)0; }
-    if constexpr (16 * G <= 32) if (maxlt > 4) { const FT t = lane_down<16 * G>(acc); acc += lt > 4 ? t : (FT)0; }
-    if constexpr (32 * G <= 32) if (maxlt > 5) { const FT t = lane_down<32 * G>(acc); acc += lt > 5 ? t : (FT)0; }
-    return acc;
-}
-
-// Reciprocal of a pivot: the FP32 factor form uses the hardware reciprocal (1 ulp),
-// the FP64 form an IEEE division.
-__device__ __forceinline__ float pivot_recip(float v) { return __builtin_amdgcn_rcpf(v); }
-__device__ __forceinline__ double pivot_recip(double v) { return 1.0 / v; }
-// v of lane `lane` (uniform over the wave) in every lane
-__device__ __forceinline__ float lane_read(float v, int lane) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
-}
-__device__ __forceinline__ double lane_read(double v, int lane) {
-    const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
-    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)b, lane);
-    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(b >> 32), lane);
-    return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
-}
-// zero or non-finite pivot (klu_refactor failure)
-template <typename FT>
-__device__ __forceinline__ bool bad_pivot(FT v) { return !(fabs(v) > (FT)0 && fabs(v) < (FT)INFINITY); }
 
 template <typename FT, int G, int NT, bool LEAN>
 __global__ void __launch_bounds__(NT) k_nr(const KArgs a) {
@@ -961,168 +773,10 @@ __global__ void __launch_bounds__(NT) k_nr(const KArgs a) {
         }
         tmark(1);
         // ---- dense tail: the m x m tile of every instance ---------------------------------
-        // Tile at slots [0, m*(m+1)): row-major with row stride m + 1, the right-hand side
-        // held as column m. Right-looking LU with diagonal pivots, four columns per pass (one
-        // barrier per pass): pass k eliminates columns k .. k+c-1 (c = min(4, m - k)) from the
-        // trailing block (rows >= k+c, columns >= k+c, the vector included) with the rank-c update
-        //   T(i,j) -= sum_q L(i,k+q) U(k+q,j),
-        //   U(k+q,j) = T(k+q,j) - sum_{r<q} L(k+q,k+r) U(k+r,j),
-        //   L(i,k+q) = (T(i,k+q) - sum_{r<q} L(i,k+r) U(k+r,k+q)) / d_k+q,
-        // every lane computing the c x c diagonal block's factors and the L and U factors of its
-        // entry from the tile. Rows k+1 .. k+c-1 of U and the c reciprocal pivots are stored one
-        // pass later (so that no pass writes what it reads); L itself is not stored, nothing
-        // after the forward sweep reads it.
-        // Then the backward sweep on the first wave alone (its lanes hold s < 64 / G of
-        // every instance; LDS accesses of one wave complete in issue order, so its passes
-        // need no barrier): x_k = y_k / d_k, y_i -= U(i,k) x_k for i < k; with one instance per
-        // workgroup, in registers.
         if (a.m > 0) {
-            const int m = a.m, ld = m + 1;
-            auto T = [&](int i, int j) -> int { return (i * ld + j) * G + g; };  // LDS index
-            // the previous pass's block: its columns, reciprocal pivots and L factors
-            int pc = 0;
-            FT pr0 = (FT)0, pr1 = (FT)0, pr2 = (FT)0, pr3 = (FT)0;
-            FT pl10 = (FT)0, pl20 = (FT)0, pl21 = (FT)0, pl30 = (FT)0, pl31 = (FT)0, pl32 = (FT)0;
-            bool bad = false;
-            for (int k = 0;; k += 4) {
-                if (act) {
-                    const int c = min(4, m - k);  // columns of this pass's block (<= 0: none)
-                    FT r0 = (FT)0, r1 = (FT)0, r2 = (FT)0, r3 = (FT)0;
-                    FT l10 = (FT)0, l20 = (FT)0, l21 = (FT)0, l30 = (FT)0, l31 = (FT)0, l32 = (FT)0;
-                    if (c > 0) {
-                        // the block's LU, in the same order in every lane
-                        FT u01 = (FT)0, u02 = (FT)0, u03 = (FT)0, u12 = (FT)0, u13 = (FT)0, u23 = (FT)0;
-                        const FT d0 = Xl[T(k, k)];
-                        bad |= bad_pivot(d0);
-                        r0 = pivot_recip(d0);
-                        if (c > 1) {
-                            u01 = Xl[T(k, k + 1)];
-                            l10 = Xl[T(k + 1, k)] * r0;
-                            const FT d1 = Xl[T(k + 1, k + 1)] - l10 * u01;
-                            bad |= bad_pivot(d1);
-                            r1 = pivot_recip(d1);
-                        }
-                        if (c > 2) {
-                            u02 = Xl[T(k, k + 2)];
-                            u12 = Xl[T(k + 1, k + 2)] - l10 * u02;
-                            l20 = Xl[T(k + 2, k)] * r0;
-                            l21 = (Xl[T(k + 2, k + 1)] - l20 * u01) * r1;
-                            const FT d2 = Xl[T(k + 2, k + 2)] - l20 * u02 - l21 * u12;
-                            bad |= bad_pivot(d2);
-                            r2 = pivot_recip(d2);
-                        }
-                        if (c > 3) {
-                            u03 = Xl[T(k, k + 3)];
-                            u13 = Xl[T(k + 1, k + 3)] - l10 * u03;
-                            u23 = Xl[T(k + 2, k + 3)] - l20 * u03 - l21 * u13;
-                            l30 = Xl[T(k + 3, k)] * r0;
-                            l31 = (Xl[T(k + 3, k + 1)] - l30 * u01) * r1;
-                            l32 = (Xl[T(k + 3, k + 2)] - l30 * u02 - l31 * u12) * r2;
-                            const FT d3 = Xl[T(k + 3, k + 3)] - l30 * u03 - l31 * u13 - l32 * u23;
-                            bad |= bad_pivot(d3);
-                            r3 = pivot_recip(d3);
-                        }
-                        // entries (i, j), i in [k+c, m), j in [k+c, m]: w rows of w + 1
-                        const int w = m - k - c, wc = w + 1;
-                        // row = floor((idx + 1/2) / wc): the fractional part of the exact
-                        // quotient stays >= 1/(2 wc) from an integer, far above the float error
-                        const float inv = __builtin_amdgcn_rcpf((float)wc);
-                        for (int idx = s; idx < w * wc; idx += nslot) {
-                            const int rr = (int)(((float)idx + 0.5f) * inv);
-                            const int i = k + c + rr, j = k + c + (idx - rr * wc);
-                            const FT li0 = Xl[T(i, k)] * r0;
-                            const FT u0j = Xl[T(k, j)];
-                            FT upd = li0 * u0j;
-                            if (c > 1) {
-                                const FT li1 = (Xl[T(i, k + 1)] - li0 * u01) * r1;
-                                const FT u1j = Xl[T(k + 1, j)] - l10 * u0j;
-                                upd += li1 * u1j;
-                                if (c > 2) {
-                                    const FT li2 = (Xl[T(i, k + 2)] - li0 * u02 - li1 * u12) * r2;
-                                    const FT u2j = Xl[T(k + 2, j)] - l20 * u0j - l21 * u1j;
-                                    upd += li2 * u2j;
-                                    if (c > 3) {
-                                        const FT li3 = (Xl[T(i, k + 3)] - li0 * u03 - li1 * u13 - li2 * u23) * r3;
-                                        const FT u3j = Xl[T(k + 3, j)] - l30 * u0j - l31 * u1j - l32 * u2j;
-                                        upd += li3 * u3j;
-                                    }
-                                }
-                            }
-                            Xl[T(i, j)] -= upd;
-                        }
-                    }
-                    if (k >= 4 && pc > 1) {  // rows p+1 .. p+pc-1 of U of the previous pass's block
-                        const int p = k - 4;
-                        for (int j = p + 2 + s; j <= m; j += nslot) {
-                            const FT u0j = Xl[T(p, j)];
-                            const FT u1j = Xl[T(p + 1, j)] - pl10 * u0j;
-                            Xl[T(p + 1, j)] = u1j;
-                            if (pc > 2 && j > p + 2) {
-                                const FT u2j = Xl[T(p + 2, j)] - pl20 * u0j - pl21 * u1j;
-                                Xl[T(p + 2, j)] = u2j;
-                                if (pc > 3 && j > p + 3)
-                                    Xl[T(p + 3, j)] = Xl[T(p + 3, j)] - pl30 * u0j - pl31 * u1j - pl32 * u2j;
-                            }
-                        }
-                    }
-                    if (k >= 4 && pc > 0 && s == 0) {  // and its reciprocal pivots
-                        const int p = k - 4;
-                        Xl[T(p, p)] = pr0;
-                        if (pc > 1) Xl[T(p + 1, p + 1)] = pr1;
-                        if (pc > 2) Xl[T(p + 2, p + 2)] = pr2;
-                        if (pc > 3) Xl[T(p + 3, p + 3)] = pr3;
-                    }
-                    pc = max(c, 0);
-                    pr0 = r0; pr1 = r1; pr2 = r2; pr3 = r3;
-                    pl10 = l10; pl20 = l20; pl21 = l21; pl30 = l30; pl31 = l31; pl32 = l32;
-                }
-                __syncthreads();
-                if (k >= m) break;
-            }
-            if (bad && s == 0) s_piv[g] = 1;
-            if (G == 1 && m <= 128) {
-                // One instance per workgroup: lane s of the first wave holds y_s and y_s+64 in
-                // registers, and x_k = y_k / d_k reaches every lane by a lane read of its owner,
-                // so a step is a few dependent register operations. U(i, k) and 1/d_k are not
-                // written by the sweep: each step's reads are issued one step ahead.
-                if (threadIdx.x < 64 && act) {
-                    FT y0 = s < m ? Xl[T(s, m)] : (FT)0, y1 = s + 64 < m ? Xl[T(s + 64, m)] : (FT)0;
-                    // column k's reads, clamped into the tile (a lane's U entries of rows i >= k
-                    // are read but not used)
-                    auto col = [&](int k, FT& u0, FT& u1, FT& dk) {
-                        const int c = max(k, 0);
-                        dk = Xl[T(c, c)];
-                        u0 = Xl[T(min(s, m - 1), c)];
-                        u1 = Xl[T(min(s + 64, m - 1), c)];
-                    };
-                    FT u0, u1, dk;
-                    col(m - 1, u0, u1, dk);
-                    for (int k = m - 1; k >= 0; --k) {
-                        FT nu0, nu1, ndk;
-                        col(k - 1, nu0, nu1, ndk);
-                        const FT xk = lane_read(k < 64 ? y0 : y1, k & 63) * dk;
-                        if (s == (k & 63)) {
-                            if (k < 64) y0 = xk;
-                            else y1 = xk;
-                        }
-                        if (s < k) y0 -= u0 * xk;  // rows i < k only: a non-finite x_k leaves the others
-                        if (s + 64 < k) y1 -= u1 * xk;
-                        u0 = nu0; u1 = nu1; dk = ndk;
-                    }
-                    if (s < m) Xl[T(s, m)] = y0;
-                    if (s + 64 < m) Xl[T(s + 64, m)] = y1;
-                }
-            } else if (threadIdx.x < 64 && act) {
-                constexpr int ws = 64 / G;  // lanes of one instance in the first wave
-                for (int k = m - 1; k >= 0; --k) {
-                    const FT xk = Xl[T(k, m)] * Xl[T(k, k)];
-                    for (int i = s; i < k; i += ws) Xl[T(i, m)] -= Xl[T(i, k)] * xk;
-                    if (s == 0) Xl[T(k, m)] = xk;
-                    // keep this pass's LDS writes ahead of the next pass's reads in the code
-                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-                }
-            }
+            bool bad_t = false;
+            dense_tail_lds<FT, G, NT>(Xl, a.m, g, s, act, bad_t);
+            if (bad_t && s == 0) s_piv[g] = 1;
             __syncthreads();
         }
         tmark(2);
@@ -1436,6 +1090,21 @@ __global__ void k_gather_y(const double* __restrict__ Y, const int2* __restrict_
     }
 }
 
+// The same for the block plan: off-diagonal entries in jagged-diagonal order, then the rows' diagonals.
+__global__ void k_gather_rows(const double* __restrict__ Y, const int* __restrict__ jd_pos, int nent,
+                              const int4* __restrict__ rows, int nrow, double* __restrict__ Yjd, double* __restrict__ Yrow) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < nent) {
+        const int p = jd_pos[i];
+        Yjd[2 * i] = Y[2 * p];
+        Yjd[2 * i + 1] = Y[2 * p + 1];
+    } else if (i < nent + nrow) {
+        const int r = i - nent, p = rows[r].z;
+        Yrow[2 * r] = Y[2 * p];
+        Yrow[2 * r + 1] = Y[2 * p + 1];
+    }
+}
+
 // The first kernel of a solve launch: zeroes the NR kernel's work-queue counter and, unless
 // the voltages are solved in place, writes the initial V of every launch instance (its first
 // row: the chain head in chain mode) from V0 (one row per instance, or one shared row).
@@ -1665,7 +1334,7 @@ struct pfgpu_grid {
     pfgpu::DevicePlan P;
     pfgpu_grid_info info{};
     DevBuf<int> yr_ptr, yr_col, yr_pos, fslot_p, fslot_q, ux_bus, ux_slot, j_ypos, j_rbus, j_cbus, j_slot, zero_slots;
-    DevBuf<int> yr_pc, yr_ell, ye_pos, ye_rc, ye_slot, ye_jidx, ye_diag_of, jc_slot, jc_jidx;
+    DevBuf<int> yr_ell, ye_pos, ye_rc, ye_slot, ye_jidx, ye_diag_of, jc_slot, jc_jidx;
     int ell_w = 0;  // columns of yr_ell
     DevBuf<double> jc_val;
     DevBuf<int8_t> ux_kind;
@@ -1678,6 +1347,22 @@ struct pfgpu_grid {
         DevBuf<int> lv_K, fs, bs;
     };
     std::vector<std::unique_ptr<Streams>> streams;  // by (G, block size, value size, lean)
+    // Block form of the factorisation (blocks.hpp), the plan of every AC and fast-decoupled solve on
+    // J's own diagonal; the scalar plan P then holds only the sizes and Ybus rows until a launch needs
+    // it (ensure_scalar_plan: wide launches)
+    struct Block {
+        pfgpu::BlockPlan P;
+        DevBuf<int> bus_y, tail_src, rows, jd_ptr, jd, jd_pos, jd_jidx, row_jidx, y_row, y_ent, jc_dst, jc_jidx;
+        DevBuf<double> jc_val;
+        struct Lanes {
+            DevBuf<int> fs, bs, f_at, b_at;
+            DevBuf<uint64_t> f_mask, b_mask;
+            int f_words, b_words;
+        };
+        std::map<int, std::unique_ptr<Lanes>> lanes;  // by (G, block size, value size)
+    };
+    std::unique_ptr<Block> blk, blk_life;  // value pairs by use; by life, for launches that overlay V (build_blocks)
+    bool scalar_plan = false;
     // autotuned launch shape per precision (G, block), 0 = not tuned
     int tuned_G[2] = {0, 0}, tuned_NT[2] = {0, 0};
     // the next solve's first iteration is the solver's first factorisation (KLULinearSolver::
@@ -1808,6 +1493,18 @@ size_t static_lds(int fsize, int G, int NT) {
     }
     cache[key] = mx;
     return mx;
+}
+
+// Static LDS of a kernel (cached).
+size_t static_lds_of(const void* fn) {
+    static std::mutex mu;
+    static std::map<const void*, size_t> cache;
+    std::lock_guard<std::mutex> lk(mu);
+    const auto it = cache.find(fn);
+    if (it != cache.end()) return it->second;
+    hipFuncAttributes attr{};
+    HIP_OK(hipFuncGetAttributes(&attr, fn));
+    return cache[fn] = attr.sharedSizeBytes;
 }
 
 size_t align16(size_t x) { return (x + 15) & ~(size_t)15; }
@@ -1946,6 +1643,15 @@ struct SolveArgs {
     long long jx_row = 0;   // the row whose J values Jx_last receives
 };
 
+// Resident workgroups of a kernel at its LDS size.
+int resident_blocks_of(const pfgpu_ctx* ctx, const void* fn, int NT, size_t lds) {
+    if (lds > 65536) HIP_OK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    int per_cu = 0;
+    HIP_OK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, NT, lds));
+    if (per_cu < 1) throw ApiError(PFGPU_E_INTERNAL, "the NR launch shape cannot be resident on a CU");
+    return per_cu * std::max(1, ctx->n_cu);
+}
+
 // Resident workgroups of a launch shape (occupancy of the kernel variant at its LDS size).
 int resident_blocks(const pfgpu_ctx* ctx, int fsize, int G, int NT, bool lean, size_t lds) {
     const void* fn;
@@ -1955,11 +1661,7 @@ int resident_blocks(const pfgpu_ctx* ctx, int fsize, int G, int NT, bool lean, s
     else
         fn = NT == 1024 ? (lean ? nr_kernel_g<double, 1024, true>(G) : nr_kernel_g<double, 1024, false>(G))
                         : (lean ? nr_kernel_g<double, 256, true>(G) : nr_kernel_g<double, 256, false>(G));
-    if (lds > 65536) HIP_OK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    int per_cu = 0;
-    HIP_OK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, NT, lds));
-    if (per_cu < 1) throw ApiError(PFGPU_E_INTERNAL, "the NR launch shape cannot be resident on a CU");
-    return per_cu * std::max(1, ctx->n_cu);
+    return resident_blocks_of(ctx, fn, NT, lds);
 }
 
 // Per-call rows in ctx->aux: [queue counter | fallback count | pad] [phase clocks: 8 x u64]
@@ -1993,7 +1695,7 @@ constexpr int kWideBlocks = 32;  // workgroups of a wide launch (PFGPU_WIDE_BLOC
 bool wide_wanted(const pfgpu_grid* gr, const SolveArgs& q, int G_req, int nunits, const FixedScratch* fx) {
     if (gr->dc || gr->fdpf || q.Jx_last || fx) return false;
     if (G_req == -1) return true;
-    return G_req == 0 && nunits == 1 && (long long)gr->P.pairs.size() / 4 >= kWidePairs;
+    return G_req == 0 && nunits == 1 && gr->info.n_pairs >= kWidePairs;
 }
 
 // log2 of the team size of each level: the largest power of two (at most 64, at most the level's
@@ -2011,8 +1713,11 @@ std::vector<int> level_teams(const std::vector<int>& lvl, const std::vector<int>
     return out;
 }
 
+void ensure_scalar_plan(pfgpu_grid* g);
+
 void launch_wide(pfgpu_ctx* ctx, pfgpu_grid* gr, const SolveArgs& q, int precision, int nunits, const int* imap,
                  const AuxLayout& AL, bool fresh, pfgpu_stats* st) {
+    ensure_scalar_plan(gr);
     const pfgpu::DevicePlan& P = gr->P;
     const int n = P.n;
     const bool fp32 = precision != PFGPU_FP64;
@@ -2099,127 +1804,9 @@ void launch_wide(pfgpu_ctx* ctx, pfgpu_grid* gr, const SolveArgs& q, int precisi
     }
 }
 
-// One NR launch (k_init_v, k_gather_y for a shared Ybus, k_nr) over `nunits` launch units;
-// imap (device, or null) maps them to the caller's instances / chains. With a fixed workspace the
-// launch allocates nothing: the schedule of its launch shape must already be on the device, and
-// the number of workgroups is capped to what the workspace holds (each workgroup takes groups of
-// instances from the work queue, so fewer workgroups only means less concurrency).
-void launch_pass(pfgpu_ctx* ctx, pfgpu_grid* gr, const SolveArgs& q, int precision, int G_req, int NT_req,
-                 int nunits, const int* imap, const AuxLayout& AL, bool fresh, pfgpu_stats* st,
-                 const FixedScratch* fx = nullptr) {
-    if (wide_wanted(gr, q, G_req, nunits, fx)) {
-        launch_wide(ctx, gr, q, precision, nunits, imap, AL, fresh, st);
-        return;
-    }
-    const pfgpu::DevicePlan& P = gr->P;
-    const int n = P.n;
-    const int fsize = precision == PFGPU_FP64 ? 8 : 4;
-    const int pslot = precision == PFGPU_FP64 ? 0 : 1;
-    if (G_req == -1) G_req = 0;  // a wide launch was not possible here (DC grid, J capture, fixed scratch)
-    if (G_req == 0 && NT_req == 0 && gr->tuned_G[pslot]) {
-        G_req = gr->tuned_G[pslot];
-        NT_req = gr->tuned_NT[pslot];
-    }
-    LaunchChoice lc = choose_launch(ctx, P, nunits, fsize, G_req, NT_req);
-    if (fx) {
-        const int ix = shape_index(lc.G, lc.NT, fsize, lc.lean);
-        if ((int)gr->streams.size() <= ix || !gr->streams[ix])
-            throw ApiError(PFGPU_E_INVALID, "the schedule of this launch shape is not on the device yet: solve a batch "
-                                            "of this shape once with pfgpu_solve_batch_device first");
-    } else {
-        ensure_streams(gr, lc.G, lc.NT, fsize, lc.lean);
-    }
-    const long long ngroups = ((long long)nunits + lc.G - 1) / lc.G;
-    int nres = (int)std::min<long long>(ngroups, resident_blocks(ctx, fsize, lc.G, lc.NT, lc.lean, lc.lds));
-    const bool gather = q.Yx_stride == 0;
-    const size_t gather_bytes = gather ? align_up((size_t)gr->ell_w * n * 16) + align_up(P.ye_pos.size() * 16) : 0;
-    if (fx) {
-        // workgroups whose rows fit the fixed workspace (4 * 256 bytes covers the roundings)
-        const size_t per_block = (size_t)lc.G * ((size_t)n * 16 + (size_t)std::max(P.nyd, 1) * 16) +
-                                 (size_t)lc.nspill * lc.G * fsize;
-        const size_t room = fx->ws_bytes > gather_bytes + 1024 ? fx->ws_bytes - gather_bytes - 1024 : 0;
-        const long long cap = per_block ? (long long)(room / per_block) : nres;
-        if (cap < 1) throw ApiError(PFGPU_E_BUDGET, "the grid's per-workgroup rows do not fit the fixed scratch");
-        nres = (int)std::min<long long>(nres, cap);
-    }
-    const long long slots = (long long)nres * lc.G;  // workspace rows: one per resident instance
-    size_t off = 0;
-    const size_t o_va = off; off += align_up((size_t)slots * n * 8);
-    const size_t o_vm = off; off += align_up((size_t)slots * n * 8);
-    const size_t o_ib = off; off += align_up((size_t)slots * std::max(P.nyd, 1) * 16);
-    const size_t o_x = off; off += align_up((size_t)nres * lc.nspill * lc.G * fsize);
-    const size_t o_yell = off; off += gather ? align_up((size_t)gr->ell_w * n * 16) : 0;
-    const size_t o_yye = off; off += gather ? align_up(P.ye_pos.size() * 16) : 0;
-    if (fx && off > fx->ws_bytes) throw ApiError(PFGPU_E_INTERNAL, "fixed scratch layout overflow");
-    char* ws = fx ? fx->ws : static_cast<char*>(ws_get(ctx, std::max<size_t>(off, 256)));
-    char* aux = fx ? fx->aux : static_cast<char*>(ctx->aux);
-    hipStream_t stream = ctx->stream;
-    int* queue = reinterpret_cast<int*>(aux + AL.o_queue);
-    unsigned long long* phase = st ? reinterpret_cast<unsigned long long*>(aux + AL.o_phase) : nullptr;
-    // in place (V0 == V, one row per instance): nothing to copy, rows are read where they are
-    const bool copy = !(q.V0 == q.V && q.v0_stride != 0 && q.chain == 1);
-    KArgs a;
-    std::memset(&a, 0, sizeof(a));  // padding too: the struct's bytes key the graph cache
-    a.n = n; a.N = P.N; a.nJ = P.nJ; a.nzero = (int)P.zero_slots.size(); a.nlev = P.nlev; a.nblev = P.nblev;
-    a.m = P.m;
-    if (lc.nlds < P.m * P.m + P.m) throw ApiError(PFGPU_E_INTERNAL, "dense tail does not fit in LDS");
-    a.nlds = lc.nlds; a.nspill = lc.nspill;
-    a.single_slack = gr->info.single_slack; a.ninst = nunits; a.max_iter = q.max_iter; a.tol = q.tol;
-    a.yr_ptr = gr->yr_ptr.p; a.yr_col = gr->yr_col.p; a.yr_pos = gr->yr_pos.p;
-    a.yr_pc = reinterpret_cast<const int2*>(gr->yr_pc.p);
-    a.yr_ell = reinterpret_cast<const int2*>(gr->yr_ell.p);
-    a.ye_pos = gr->ye_pos.p; a.ye_rc = reinterpret_cast<const int2*>(gr->ye_rc.p);
-    a.ye_slot = reinterpret_cast<const int4*>(gr->ye_slot.p); a.ye_jidx = reinterpret_cast<const int4*>(gr->ye_jidx.p);
-    a.nye = (int)P.ye_pos.size();
-    a.jc_slot = gr->jc_slot.p; a.jc_jidx = gr->jc_jidx.p; a.jc_val = gr->jc_val.p; a.njc = (int)P.jc_slot.size();
-    a.dptr = q.dptr; a.dpos = q.dpos; a.dval = q.dval;
-    a.fslot_p = gr->fslot_p.p; a.fslot_q = gr->fslot_q.p;
-    a.ux_bus = gr->ux_bus.p; a.ux_slot = gr->ux_slot.p; a.ux_kind = gr->ux_kind.p;
-    a.bus_dx = reinterpret_cast<const int2*>(gr->bus_dx.p); a.slack_dx = gr->slack_dx;
-    a.j_ypos = gr->j_ypos.p; a.j_rbus = gr->j_rbus.p; a.j_cbus = gr->j_cbus.p; a.j_sel = gr->j_sel.p; a.j_cval = gr->j_cval.p;
-    a.j_slot = gr->j_slot.p; a.zero_slots = gr->zero_slots.p;
-    const auto& ls = *gr->streams[shape_index(lc.G, lc.NT, fsize, lc.lean)];
-    a.lv_K = ls.lv_K.p; a.lvk_off = (int)lc.lvk_off; a.sh_off = (int)lc.sh_off;
-    a.fs = reinterpret_cast<const int4*>(ls.fs.p); a.bs = reinterpret_cast<const int4*>(ls.bs.p);
-    a.w = gr->w.p;
-    a.Yx = q.Yx; a.y_stride = (long long)q.Yx_stride * 2;
-    a.S = q.S; a.s_stride = (long long)q.sbus_stride * 2;
-    a.V = q.V; a.Va = reinterpret_cast<double*>(ws + o_va); a.Vm = reinterpret_cast<double*>(ws + o_vm);
-    a.Ib = reinterpret_cast<double*>(ws + o_ib); a.Xg = ws + o_x;
-    a.ye_diag_of = gr->ye_diag_of.p; a.nyd = P.nyd;
-    a.iters = q.iters; a.status = q.status; a.Jx_last = q.Jx_last; a.jx_row = q.jx_row;
-    a.v_off = (int)lc.v_off;
-    a.Yell = gather ? reinterpret_cast<const double*>(ws + o_yell) : nullptr;
-    a.Yye = gather ? reinterpret_cast<const double*>(ws + o_yye) : nullptr;
-    a.imap = imap;
-    a.chain = q.chain;
-    a.nrows = q.nrows;
-    a.fresh = fresh ? 1 : 0;
-    a.stall_tol = std::sqrt(q.tol);
-    a.growth_tau = fsize == 4 ? 1.0 / 1024.0 : 1e-10;
-    a.flags = reinterpret_cast<int*>(aux + AL.o_flags);
-    a.phase_t = phase;
-    a.queue = queue;
-    a.ngroups = ngroups;
-    a.dc = gr->dc ? 1 : 0;
-    a.slack0 = P.slack0;
-    a.fdpf = gr->fdpf ? 1 : 0;
-    if (gr->dc) a.max_iter = 1;
-    const int nell = gr->ell_w * n, nye = (int)P.ye_pos.size();
-    auto issue = [&]() {
-        hipLaunchKernelGGL(k_init_v, dim3(copy ? 1024 : 1), dim3(256), 0, stream, q.V0, (long long)q.v0_stride * 2, q.V,
-                           n, nunits, imap, q.chain, queue, phase, copy ? 1 : 0);
-        HIP_OK(hipGetLastError());
-        if (gather) {
-            hipLaunchKernelGGL(k_gather_y, dim3((nell + nye + 255) / 256), dim3(256), 0, stream, q.Yx, a.yr_ell, nell,
-                               a.ye_pos, nye, reinterpret_cast<double*>(ws + o_yell),
-                               reinterpret_cast<double*>(ws + o_yye));
-            HIP_OK(hipGetLastError());
-        }
-        if (fsize == 4) launch_nr_any<float>(lc.G, lc.NT, lc.lean, a, nres, lc.lds, stream);
-        else launch_nr_any<double>(lc.G, lc.NT, lc.lean, a, nres, lc.lds, stream);
-    };
-    // the launch sequence's key: every argument of the three launches
+// What identifies a launch sequence (k_init_v, k_gather_y and the NR kernel): every argument of the three.
+std::vector<unsigned char> sequence_key(const void* args, size_t bytes, const SolveArgs& q, bool copy, int nres, int G,
+                                        int NT, bool lean, int fsize, bool gather, size_t lds) {
     struct Extra {
         const double* V0;
         long long v0s;
@@ -2227,11 +1814,24 @@ void launch_pass(pfgpu_ctx* ctx, pfgpu_grid* gr, const SolveArgs& q, int precisi
         size_t lds;
     } ex;
     std::memset(&ex, 0, sizeof(ex));
-    ex.V0 = q.V0; ex.v0s = (long long)q.v0_stride * 2; ex.copy = copy; ex.nres = nres; ex.G = lc.G; ex.NT = lc.NT;
-    ex.lean = lc.lean; ex.fsize = fsize; ex.gather = gather; ex.lds = lc.lds;
-    std::vector<unsigned char> key(sizeof(KArgs) + sizeof(Extra));
-    std::memcpy(key.data(), &a, sizeof(KArgs));
-    std::memcpy(key.data() + sizeof(KArgs), &ex, sizeof(Extra));
+    ex.V0 = q.V0; ex.v0s = (long long)q.v0_stride * 2; ex.copy = copy; ex.nres = nres; ex.G = G; ex.NT = NT;
+    ex.lean = lean; ex.fsize = fsize; ex.gather = gather; ex.lds = lds;
+    std::vector<unsigned char> key(bytes + sizeof(Extra));
+    std::memcpy(key.data(), args, bytes);
+    std::memcpy(key.data() + bytes, &ex, sizeof(Extra));
+    return key;
+}
+
+struct LaunchShape {
+    int G, NT, slots, nres;
+    long long ngroups;
+};
+
+// Issues a launch sequence, or replays its captured graph, waits for it and fills the stats.
+template <class Issue>
+void run_sequence(pfgpu_ctx* ctx, pfgpu_grid* gr, std::vector<unsigned char> key, Issue&& issue, const FixedScratch* fx,
+                  const unsigned long long* phase, const LaunchShape& sh, pfgpu_stats* st) {
+    hipStream_t stream = ctx->stream;
     static const bool graphs_on = [] {
         const char* e = std::getenv("PFGPU_GRAPH");
         return !(e && e[0] == '0');
@@ -2288,17 +1888,318 @@ void launch_pass(pfgpu_ctx* ctx, pfgpu_grid* gr, const SolveArgs& q, int precisi
         float ms = 0;
         HIP_OK(hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
         st->kernel_s += ms * 1e-3;
-        st->instances_per_wg = lc.G;
-        st->block_size = lc.NT;
-        st->lds_slots = lc.nlds;
-        st->workgroups = (int)std::min<long long>(ngroups, INT_MAX);
-        st->resident_workgroups = nres;
+        st->instances_per_wg = sh.G;
+        st->block_size = sh.NT;
+        st->lds_slots = sh.slots;
+        st->workgroups = (int)std::min<long long>(sh.ngroups, INT_MAX);
+        st->resident_workgroups = sh.nres;
         st->graph_launches += replayed ? 1 : 0;
         unsigned long long ph[8];
         HIP_OK(hipMemcpyAsync(ph, phase, sizeof(ph), hipMemcpyDeviceToHost, stream));
         HIP_OK(hipStreamSynchronize(stream));
         for (int k = 0; k < 6; ++k) st->phase_s[k] += (double)ph[k] / ctx->wall_hz;
     }
+}
+
+// ---------------------------------------------------------------------------
+// Launches on the block plan
+// ---------------------------------------------------------------------------
+struct BlockChoice {
+    int G, NT, nlds, nspill;
+    bool lean;
+    size_t lds, sh_off;
+    long long v_off;  // -1: V in global memory
+};
+
+// Launch heuristic: the largest G whose values and V fit entirely in LDS while keeping at least two
+// workgroups per CU; otherwise G = 1 with the most used pairs in LDS and the rest spilled. One workgroup
+// of 1024 lanes when its values take more than half of the LDS, else workgroups of 256.
+BlockChoice choose_block(const pfgpu_ctx* ctx, const pfgpu_grid::Block& b, int ninst, int fsize, int G_req, int NT_req) {
+    const pfgpu::BlockPlan& P = b.P;
+    auto avail = [&](int G, int NT) -> size_t {
+        const size_t fixed = pfgpu_block::state_bytes(G, NT) + 32;
+        return (size_t)ctx->lds_max > fixed ? (size_t)ctx->lds_max - fixed : 0;
+    };
+    auto values = [&](int G) -> size_t { return (size_t)P.npairs * 2 * G * fsize; };
+    const size_t fixed_pairs = (size_t)P.tile_pairs + 2;  // always in LDS
+    BlockChoice c{};
+    c.G = 1;
+    const long long ncu = std::max(1, ctx->n_cu);
+    if (G_req > 0) {
+        c.G = G_req;
+    } else {
+        for (int G = kMaxG; G >= 2; G >>= 1)
+            if (values(G) + (size_t)P.n * G * 16 <= avail(G, 1024) && (ninst + G - 1) / G >= 2 * ncu) { c.G = G; break; }
+    }
+    while (c.G > 1 && fixed_pairs * 2 * c.G * fsize > avail(c.G, 1024)) c.G >>= 1;
+    c.NT = values(c.G) > avail(c.G, 1024) / 2 ? 1024 : 256;
+    if (NT_req == 256 || NT_req == 1024) c.NT = NT_req;
+    const size_t room = avail(c.G, c.NT), pair = (size_t)2 * c.G * fsize;
+    c.nlds = (int)std::min<size_t>((size_t)P.npairs, room / pair);
+    while (c.nlds < P.npairs && c.nlds > 0 && P.second[c.nlds]) --c.nlds;  // between two blocks
+    if ((size_t)c.nlds < fixed_pairs) throw ApiError(PFGPU_E_INVALID, "the grid's dense tail does not fit in LDS");
+    c.nspill = P.npairs - c.nlds;
+    c.lean = c.nspill == 0;
+    // V in LDS: after the values, or, with every value in LDS, over the ones that are not in use while J is
+    // assembled (the order by life keeps those last); the workgroup state follows
+    const size_t state = pfgpu_block::state_bytes(c.G, c.NT), v = (size_t)P.n * c.G * 16;
+    size_t end = align16((size_t)c.nlds * pair);
+    c.v_off = -1;
+    if (end + v + state <= (size_t)ctx->lds_max) {
+        c.v_off = (long long)end;
+        end += v;
+    } else if (c.lean && P.fill_at < P.npairs && align16((size_t)P.fill_at * pair) + v + state <= (size_t)ctx->lds_max) {
+        c.v_off = (long long)align16((size_t)P.fill_at * pair);
+        end = std::max(end, align16((size_t)c.v_off + v));
+    }
+    c.sh_off = end;
+    c.lds = end + state;
+    return c;
+}
+
+pfgpu_grid::Block::Lanes& block_lanes(pfgpu_grid::Block& b, const BlockChoice& c, int fsize, bool may_build) {
+    auto& slot = b.lanes[(c.G * 2 + (c.NT == 1024 ? 1 : 0)) * 2 + (fsize == 8 ? 1 : 0)];
+    if (!slot) {
+        if (!may_build)
+            throw ApiError(PFGPU_E_INVALID, "the schedule of this launch shape is not on the device yet: solve a batch "
+                                            "of this shape once with pfgpu_solve_batch_device first");
+        const pfgpu::BlockStreams S = pfgpu::build_block_streams(b.P, c.G, c.NT / 64, fsize, c.nlds);
+        auto t = std::make_unique<pfgpu_grid::Block::Lanes>();
+        t->fs.upload(S.fs);
+        t->bs.upload(S.bs);
+        t->f_at.upload(S.f_at);
+        t->b_at.upload(S.b_at);
+        t->f_mask.upload(S.f_mask);
+        t->b_mask.upload(S.b_mask);
+        t->f_words = S.f_words;
+        t->b_words = S.b_words;
+        slot = std::move(t);
+    }
+    return *slot;
+}
+
+std::unique_ptr<pfgpu_grid::Block> upload_blocks(const pfgpu_grid* g, const std::vector<int>& perm, pfgpu::BlockOrder order);
+
+// One NR launch on the block plan; as launch_pass otherwise.
+void launch_block(pfgpu_ctx* ctx, pfgpu_grid* gr, const SolveArgs& q, int precision, int G_req, int NT_req, int nunits,
+                  const int* imap, const AuxLayout& AL, bool fresh, pfgpu_stats* st, const FixedScratch* fx) {
+    const int fsize = precision == PFGPU_FP64 ? 8 : 4;
+    BlockChoice c = choose_block(ctx, *gr->blk, nunits, fsize, G_req, NT_req);
+    pfgpu_grid::Block* use = gr->blk.get();
+    if (c.lean && c.v_off < 0) {  // V does not fit beside the values: over some of them?
+        if (!gr->blk_life && !fx) gr->blk_life = upload_blocks(gr, pfgpu::column_order(gr->J), pfgpu::kByLife);
+        if (gr->blk_life) {
+            const BlockChoice cl = choose_block(ctx, *gr->blk_life, nunits, fsize, c.G, c.NT);
+            if (cl.v_off >= 0) {
+                c = cl;
+                use = gr->blk_life.get();
+            }
+        }
+    }
+    pfgpu_grid::Block& b = *use;
+    const pfgpu::BlockPlan& P = b.P;
+    const int n = P.n;
+    pfgpu_grid::Block::Lanes& ln = block_lanes(b, c, fsize, fx == nullptr);
+    const long long ngroups = ((long long)nunits + c.G - 1) / c.G;
+    const void* fn = pfgpu_block::kernel(fsize, c.G, c.NT, c.lean);
+    if (static_lds_of(fn) != 0)  // units carry LDS addresses: the values must start at address 0
+        throw ApiError(PFGPU_E_INTERNAL, "the NR kernel has static LDS: unit offsets would not be LDS addresses");
+    int nres = (int)std::min<long long>(ngroups, resident_blocks_of(ctx, fn, c.NT, c.lds));
+    const int nrow = (int)P.row_len.size(), nent = (int)P.jd_pos.size();
+    const bool gather = q.Yx_stride == 0;
+    const size_t o_yrow = align_up((size_t)std::max(nent, 1) * 16);
+    const size_t gather_bytes = gather ? o_yrow + align_up((size_t)std::max(nrow, 1) * 16) : 0;
+    if (fx) {
+        // workgroups whose rows fit the fixed workspace (4 * 256 bytes covers the roundings)
+        const size_t per_block = (size_t)c.G * n * 16 + (size_t)c.nspill * 2 * c.G * fsize;
+        const size_t room = fx->ws_bytes > gather_bytes + 1024 ? fx->ws_bytes - gather_bytes - 1024 : 0;
+        const long long cap = per_block ? (long long)(room / per_block) : nres;
+        if (cap < 1) throw ApiError(PFGPU_E_BUDGET, "the grid's per-workgroup rows do not fit the fixed scratch");
+        nres = (int)std::min<long long>(nres, cap);
+    }
+    const long long slots = (long long)nres * c.G;
+    size_t off = 0;
+    const size_t o_va = off; off += align_up((size_t)slots * n * 8);
+    const size_t o_vm = off; off += align_up((size_t)slots * n * 8);
+    const size_t o_x = off; off += align_up((size_t)nres * c.nspill * 2 * c.G * fsize);
+    const size_t o_y = off; off += gather_bytes;
+    const size_t o_vp = off; off += q.Jx_last ? align_up((size_t)n * 16) : 0;
+    if (fx && off > fx->ws_bytes) throw ApiError(PFGPU_E_INTERNAL, "fixed scratch layout overflow");
+    char* ws = fx ? fx->ws : static_cast<char*>(ws_get(ctx, std::max<size_t>(off, 256)));
+    char* aux = fx ? fx->aux : static_cast<char*>(ctx->aux);
+    hipStream_t stream = ctx->stream;
+    int* queue = reinterpret_cast<int*>(aux + AL.o_queue);
+    unsigned long long* phase = st ? reinterpret_cast<unsigned long long*>(aux + AL.o_phase) : nullptr;
+    const bool copy = !(q.V0 == q.V && q.v0_stride != 0 && q.chain == 1);
+    pfgpu_block::BArgs a;
+    std::memset(&a, 0, sizeof(a));  // padding too: the struct's bytes key the graph cache
+    a.n = n; a.nlev = P.nlev; a.nblev = P.nblev; a.m = P.m; a.zpair = P.zpair; a.nlds = c.nlds; a.nspill = c.nspill;
+    a.single_slack = gr->info.single_slack; a.ninst = nunits; a.max_iter = q.max_iter; a.fresh = fresh ? 1 : 0;
+    a.fdpf = gr->fdpf ? 1 : 0; a.chain = q.chain;
+    a.nrow = nrow; a.nent = nent; a.njd = (int)P.jd_ptr.size(); a.njc = (int)P.jc_dst.size(); a.slack_x = P.slack_x;
+    a.slack_bus = P.slack_bus;
+    a.nnzY = gr->P.nnzY;
+    a.sh_off = (int)c.sh_off; a.v_off = (int)c.v_off;
+    a.tol = q.tol; a.stall_tol = std::sqrt(q.tol); a.growth_tau = fsize == 4 ? 1.0 / 1024.0 : 1e-10;
+    a.bus_y = b.bus_y.p; a.tail_src = b.tail_src.p; a.y_row = b.y_row.p; a.y_ent = b.y_ent.p;
+    a.rows = reinterpret_cast<const int4*>(b.rows.p); a.jd_ptr = b.jd_ptr.p; a.jd = reinterpret_cast<const int2*>(b.jd.p);
+    a.jd_pos = b.jd_pos.p; a.jd_jidx = reinterpret_cast<const int4*>(b.jd_jidx.p);
+    a.row_jidx = reinterpret_cast<const int4*>(b.row_jidx.p);
+    a.jc_dst = b.jc_dst.p; a.jc_jidx = reinterpret_cast<const int4*>(b.jc_jidx.p); a.jc_val = b.jc_val.p;
+    a.fs = reinterpret_cast<const int4*>(ln.fs.p); a.bs = reinterpret_cast<const int4*>(ln.bs.p);
+    a.f_at = ln.f_at.p; a.b_at = ln.b_at.p; a.f_words = ln.f_words; a.b_words = ln.b_words;
+    a.f_mask = reinterpret_cast<const unsigned long long*>(ln.f_mask.p);
+    a.b_mask = reinterpret_cast<const unsigned long long*>(ln.b_mask.p);
+    a.Yjd = gather ? reinterpret_cast<const double*>(ws + o_y) : nullptr;
+    a.Yrow = gather ? reinterpret_cast<const double*>(ws + o_y + o_yrow) : nullptr;
+    a.Vprev = q.Jx_last ? reinterpret_cast<double*>(ws + o_vp) : nullptr;
+    a.w = gr->w.p; a.Yx = q.Yx; a.y_stride = (long long)q.Yx_stride * 2;
+    a.dptr = q.dptr; a.dpos = q.dpos; a.dval = q.dval; a.S = q.S; a.s_stride = (long long)q.sbus_stride * 2;
+    a.V = q.V; a.Va = reinterpret_cast<double*>(ws + o_va); a.Vm = reinterpret_cast<double*>(ws + o_vm);
+    a.Xg = ws + o_x;
+    a.iters = q.iters; a.status = q.status; a.flags = reinterpret_cast<int*>(aux + AL.o_flags);
+    a.Jx_last = q.Jx_last; a.jx_row = q.jx_row; a.imap = imap; a.nrows = q.nrows; a.phase_t = phase; a.queue = queue;
+    a.ngroups = ngroups;
+    auto issue = [&]() {
+        hipLaunchKernelGGL(k_init_v, dim3(copy ? 1024 : 1), dim3(256), 0, stream, q.V0, (long long)q.v0_stride * 2, q.V,
+                           n, nunits, imap, q.chain, queue, phase, copy ? 1 : 0);
+        HIP_OK(hipGetLastError());
+        if (gather) {
+            hipLaunchKernelGGL(k_gather_rows, dim3((nent + nrow + 255) / 256), dim3(256), 0, stream, q.Yx, b.jd_pos.p, nent,
+                               a.rows, nrow, reinterpret_cast<double*>(ws + o_y), reinterpret_cast<double*>(ws + o_y + o_yrow));
+            HIP_OK(hipGetLastError());
+        }
+        pfgpu_block::launch(a, fsize, c.G, c.NT, c.lean, nres, c.lds, stream);
+    };
+    run_sequence(ctx, gr, sequence_key(&a, sizeof(a), q, copy, nres, c.G, c.NT, c.lean, fsize, gather, c.lds), issue, fx,
+                 phase, {c.G, c.NT, 2 * c.nlds, nres, ngroups}, st);
+}
+
+// One NR launch (k_init_v, k_gather_y for a shared Ybus, k_nr) over `nunits` launch units;
+// imap (device, or null) maps them to the caller's instances / chains. With a fixed workspace the
+// launch allocates nothing: the schedule of its launch shape must already be on the device, and
+// the number of workgroups is capped to what the workspace holds (each workgroup takes groups of
+// instances from the work queue, so fewer workgroups only means less concurrency).
+void launch_pass(pfgpu_ctx* ctx, pfgpu_grid* gr, const SolveArgs& q, int precision, int G_req, int NT_req,
+                 int nunits, const int* imap, const AuxLayout& AL, bool fresh, pfgpu_stats* st,
+                 const FixedScratch* fx = nullptr) {
+    if (wide_wanted(gr, q, G_req, nunits, fx)) {
+        launch_wide(ctx, gr, q, precision, nunits, imap, AL, fresh, st);
+        return;
+    }
+    const pfgpu::DevicePlan& P = gr->P;
+    const int n = P.n;
+    const int fsize = precision == PFGPU_FP64 ? 8 : 4;
+    const int pslot = precision == PFGPU_FP64 ? 0 : 1;
+    if (G_req == -1) G_req = 0;  // a wide launch was not possible here (DC grid, J capture, fixed scratch)
+    if (G_req == 0 && NT_req == 0 && gr->tuned_G[pslot]) {
+        G_req = gr->tuned_G[pslot];
+        NT_req = gr->tuned_NT[pslot];
+    }
+    if (gr->blk) {
+        launch_block(ctx, gr, q, precision, G_req, NT_req, nunits, imap, AL, fresh, st, fx);
+        return;
+    }
+    LaunchChoice lc = choose_launch(ctx, P, nunits, fsize, G_req, NT_req);
+    if (fx) {
+        const int ix = shape_index(lc.G, lc.NT, fsize, lc.lean);
+        if ((int)gr->streams.size() <= ix || !gr->streams[ix])
+            throw ApiError(PFGPU_E_INVALID, "the schedule of this launch shape is not on the device yet: solve a batch "
+                                            "of this shape once with pfgpu_solve_batch_device first");
+    } else {
+        ensure_streams(gr, lc.G, lc.NT, fsize, lc.lean);
+    }
+    const long long ngroups = ((long long)nunits + lc.G - 1) / lc.G;
+    int nres = (int)std::min<long long>(ngroups, resident_blocks(ctx, fsize, lc.G, lc.NT, lc.lean, lc.lds));
+    const bool gather = q.Yx_stride == 0;
+    const size_t gather_bytes = gather ? align_up((size_t)gr->ell_w * n * 16) + align_up(P.ye_pos.size() * 16) : 0;
+    if (fx) {
+        // workgroups whose rows fit the fixed workspace (4 * 256 bytes covers the roundings)
+        const size_t per_block = (size_t)lc.G * ((size_t)n * 16 + (size_t)std::max(P.nyd, 1) * 16) +
+                                 (size_t)lc.nspill * lc.G * fsize;
+        const size_t room = fx->ws_bytes > gather_bytes + 1024 ? fx->ws_bytes - gather_bytes - 1024 : 0;
+        const long long cap = per_block ? (long long)(room / per_block) : nres;
+        if (cap < 1) throw ApiError(PFGPU_E_BUDGET, "the grid's per-workgroup rows do not fit the fixed scratch");
+        nres = (int)std::min<long long>(nres, cap);
+    }
+    const long long slots = (long long)nres * lc.G;  // workspace rows: one per resident instance
+    size_t off = 0;
+    const size_t o_va = off; off += align_up((size_t)slots * n * 8);
+    const size_t o_vm = off; off += align_up((size_t)slots * n * 8);
+    const size_t o_ib = off; off += align_up((size_t)slots * std::max(P.nyd, 1) * 16);
+    const size_t o_x = off; off += align_up((size_t)nres * lc.nspill * lc.G * fsize);
+    const size_t o_yell = off; off += gather ? align_up((size_t)gr->ell_w * n * 16) : 0;
+    const size_t o_yye = off; off += gather ? align_up(P.ye_pos.size() * 16) : 0;
+    if (fx && off > fx->ws_bytes) throw ApiError(PFGPU_E_INTERNAL, "fixed scratch layout overflow");
+    char* ws = fx ? fx->ws : static_cast<char*>(ws_get(ctx, std::max<size_t>(off, 256)));
+    char* aux = fx ? fx->aux : static_cast<char*>(ctx->aux);
+    hipStream_t stream = ctx->stream;
+    int* queue = reinterpret_cast<int*>(aux + AL.o_queue);
+    unsigned long long* phase = st ? reinterpret_cast<unsigned long long*>(aux + AL.o_phase) : nullptr;
+    // in place (V0 == V, one row per instance): nothing to copy, rows are read where they are
+    const bool copy = !(q.V0 == q.V && q.v0_stride != 0 && q.chain == 1);
+    KArgs a;
+    std::memset(&a, 0, sizeof(a));  // padding too: the struct's bytes key the graph cache
+    a.n = n; a.N = P.N; a.nJ = P.nJ; a.nzero = (int)P.zero_slots.size(); a.nlev = P.nlev; a.nblev = P.nblev;
+    a.m = P.m;
+    if (lc.nlds < P.m * P.m + P.m) throw ApiError(PFGPU_E_INTERNAL, "dense tail does not fit in LDS");
+    a.nlds = lc.nlds; a.nspill = lc.nspill;
+    a.single_slack = gr->info.single_slack; a.ninst = nunits; a.max_iter = q.max_iter; a.tol = q.tol;
+    a.yr_ptr = gr->yr_ptr.p; a.yr_col = gr->yr_col.p; a.yr_pos = gr->yr_pos.p;
+    a.yr_ell = reinterpret_cast<const int2*>(gr->yr_ell.p);
+    a.ye_pos = gr->ye_pos.p; a.ye_rc = reinterpret_cast<const int2*>(gr->ye_rc.p);
+    a.ye_slot = reinterpret_cast<const int4*>(gr->ye_slot.p); a.ye_jidx = reinterpret_cast<const int4*>(gr->ye_jidx.p);
+    a.nye = (int)P.ye_pos.size();
+    a.jc_slot = gr->jc_slot.p; a.jc_jidx = gr->jc_jidx.p; a.jc_val = gr->jc_val.p; a.njc = (int)P.jc_slot.size();
+    a.dptr = q.dptr; a.dpos = q.dpos; a.dval = q.dval;
+    a.fslot_p = gr->fslot_p.p; a.fslot_q = gr->fslot_q.p;
+    a.ux_bus = gr->ux_bus.p; a.ux_slot = gr->ux_slot.p; a.ux_kind = gr->ux_kind.p;
+    a.bus_dx = reinterpret_cast<const int2*>(gr->bus_dx.p); a.slack_dx = gr->slack_dx;
+    a.j_ypos = gr->j_ypos.p; a.j_rbus = gr->j_rbus.p; a.j_cbus = gr->j_cbus.p; a.j_sel = gr->j_sel.p; a.j_cval = gr->j_cval.p;
+    a.j_slot = gr->j_slot.p; a.zero_slots = gr->zero_slots.p;
+    const auto& ls = *gr->streams[shape_index(lc.G, lc.NT, fsize, lc.lean)];
+    a.lv_K = ls.lv_K.p; a.lvk_off = (int)lc.lvk_off; a.sh_off = (int)lc.sh_off;
+    a.fs = reinterpret_cast<const int4*>(ls.fs.p); a.bs = reinterpret_cast<const int4*>(ls.bs.p);
+    a.w = gr->w.p;
+    a.Yx = q.Yx; a.y_stride = (long long)q.Yx_stride * 2;
+    a.S = q.S; a.s_stride = (long long)q.sbus_stride * 2;
+    a.V = q.V; a.Va = reinterpret_cast<double*>(ws + o_va); a.Vm = reinterpret_cast<double*>(ws + o_vm);
+    a.Ib = reinterpret_cast<double*>(ws + o_ib); a.Xg = ws + o_x;
+    a.ye_diag_of = gr->ye_diag_of.p; a.nyd = P.nyd;
+    a.iters = q.iters; a.status = q.status; a.Jx_last = q.Jx_last; a.jx_row = q.jx_row;
+    a.v_off = (int)lc.v_off;
+    a.Yell = gather ? reinterpret_cast<const double*>(ws + o_yell) : nullptr;
+    a.Yye = gather ? reinterpret_cast<const double*>(ws + o_yye) : nullptr;
+    a.imap = imap;
+    a.chain = q.chain;
+    a.nrows = q.nrows;
+    a.fresh = fresh ? 1 : 0;
+    a.stall_tol = std::sqrt(q.tol);
+    a.growth_tau = fsize == 4 ? 1.0 / 1024.0 : 1e-10;
+    a.flags = reinterpret_cast<int*>(aux + AL.o_flags);
+    a.phase_t = phase;
+    a.queue = queue;
+    a.ngroups = ngroups;
+    a.dc = gr->dc ? 1 : 0;
+    a.slack0 = P.slack0;
+    a.fdpf = gr->fdpf ? 1 : 0;
+    if (gr->dc) a.max_iter = 1;
+    const int nell = gr->ell_w * n, nye = (int)P.ye_pos.size();
+    auto issue = [&]() {
+        hipLaunchKernelGGL(k_init_v, dim3(copy ? 1024 : 1), dim3(256), 0, stream, q.V0, (long long)q.v0_stride * 2, q.V,
+                           n, nunits, imap, q.chain, queue, phase, copy ? 1 : 0);
+        HIP_OK(hipGetLastError());
+        if (gather) {
+            hipLaunchKernelGGL(k_gather_y, dim3((nell + nye + 255) / 256), dim3(256), 0, stream, q.Yx, a.yr_ell, nell,
+                               a.ye_pos, nye, reinterpret_cast<double*>(ws + o_yell),
+                               reinterpret_cast<double*>(ws + o_yye));
+            HIP_OK(hipGetLastError());
+        }
+        if (fsize == 4) launch_nr_any<float>(lc.G, lc.NT, lc.lean, a, nres, lc.lds, stream);
+        else launch_nr_any<double>(lc.G, lc.NT, lc.lean, a, nres, lc.lds, stream);
+    };
+    run_sequence(ctx, gr, sequence_key(&a, sizeof(a), q, copy, nres, lc.G, lc.NT, lc.lean, fsize, gather, lc.lds), issue,
+                 fx, phase, {lc.G, lc.NT, lc.nlds, nres, ngroups}, st);
 }
 
 // Computes the grid's symbolic factor, schedule and device plan from g->Y and g->J (elimination
@@ -2710,41 +2611,93 @@ int pfgpu_grid_load_fdpf(pfgpu_ctx* ctx, int n, const int* Yp, const int* Yi, co
 }
 
 namespace {
-void build_plan(pfgpu_grid* g, const std::vector<int>* perm) {
+void upload_rows(pfgpu_grid* g) {
+    const auto& P = g->P;
+    g->yr_ptr.upload(P.yr_ptr); g->yr_col.upload(P.yr_col); g->yr_pos.upload(P.yr_pos);
+    // column-major row table, width the longest row rounded up to kEll columns
+    const int n = (int)P.yr_ptr.size() - 1;
+    int w = 1;
+    for (int r = 0; r < n; ++r) w = std::max(w, P.yr_ptr[r + 1] - P.yr_ptr[r]);
+    w = (w + kEll - 1) / kEll * kEll;
+    g->ell_w = w;
+    std::vector<int> ell(2 * (size_t)w * std::max(n, 1), 0);
+    for (int r = 0; r < n; ++r)
+        for (int k = 0; k < w; ++k) {
+            const int q = P.yr_ptr[r] + k;
+            const bool in = q < P.yr_ptr[r + 1];
+            ell[2 * ((size_t)k * n + r)] = in ? P.yr_pos[q] : -1;
+            ell[2 * ((size_t)k * n + r) + 1] = in ? P.yr_col[q] : r;
+        }
+    g->yr_ell.upload(ell);
+    g->w.upload(g->w_h);
+}
+
+// A block plan and its tables on the device.
+std::unique_ptr<pfgpu_grid::Block> upload_blocks(const pfgpu_grid* g, const std::vector<int>& perm, pfgpu::BlockOrder order) {
+    auto b = std::make_unique<pfgpu_grid::Block>();
+    b->P = pfgpu::build_block_plan(g->Y, g->J, perm, order);
+    const pfgpu::BlockPlan& B = b->P;
+    if (!pfgpu::block_plan_fits(B)) return nullptr;
+    auto up = [](auto& d, auto v) {
+        if (v.empty()) v.resize(4);
+        d.upload(v);
+    };
+    b->bus_y.upload(B.bus_y);
+    up(b->tail_src, B.tail_src);
+    b->y_row.upload(g->Y.i);
+    const int nrow = (int)B.row_len.size(), nent = (int)B.jd_pos.size();
+    std::vector<int> ptr = B.jd_ptr, ent(g->Y.i.size(), -1);
+    ptr.push_back(nent);
+    for (int e = 0; e < nent; ++e) ent[B.jd_pos[e]] = e;
+    for (int i = 0; i < nrow; ++i) ent[B.rows[4 * i + 2]] = nent + i;
+    up(b->rows, B.rows); up(b->jd_ptr, ptr); up(b->jd, B.jd); up(b->jd_pos, B.jd_pos); up(b->jd_jidx, B.jd_jidx);
+    up(b->row_jidx, B.row_jidx); b->y_ent.upload(ent);
+    up(b->jc_dst, B.jc_dst); up(b->jc_jidx, B.jc_jidx); up(b->jc_val, B.jc_val);
+    return b;
+}
+
+// The block plan of a grid; P keeps the sizes and the Ybus row view. (A grid with more values than the
+// target words can name keeps the scalar plan.)
+void build_blocks(pfgpu_grid* g) {
+    const std::vector<int> perm = pfgpu::column_order(g->J);
+    g->blk = upload_blocks(g, perm, pfgpu::kByUse);
+    if (!g->blk) return;
+    const pfgpu::BlockPlan& B = g->blk->P;
+    pfgpu::DevicePlan& P = g->P;
+    const int n = g->Y.n;
+    P.n = n; P.N = g->J.N; P.nnzY = g->Y.p[n]; P.nJ = (int)g->J.Ji.size(); P.slack0 = g->J.slack0;
+    pfgpu::ybus_rows(g->Y, P);
+    upload_rows(g);
+    const pfgpu::FactorCounts fc = pfgpu::factor_counts(g->J, perm);
+    g->info.n_bus = n;
+    g->info.n_jac = P.N;
+    g->info.nnz_ybus = P.nnzY;
+    g->info.nnz_jac = P.nJ;
+    g->info.nnz_lu = fc.nnzLU;
+    g->info.n_slots = 2 * B.npairs;
+    g->info.n_levels = B.nlev;
+    g->info.n_back_levels = B.nblev;
+    g->info.n_pairs = fc.npairs;
+    g->info.flops = fc.flops;
+}
+
+void build_scalar(pfgpu_grid* g, const std::vector<int>* perm, bool rows) {
     pfgpu::SymbolicLU S = pfgpu::symbolic_lu(g->J, 96, perm);
     pfgpu::Schedule sch = pfgpu::build_schedule(S);
     g->P = pfgpu::build_device_plan(g->Y, g->J, S, sch);
     const auto& P = g->P;
-    g->info.n_bus = g->Y.n;
-    g->info.n_jac = P.N;
-    g->info.nnz_ybus = P.nnzY;
-    g->info.nnz_jac = P.nJ;
-    g->info.nnz_lu = P.nnzLU;
-    g->info.n_slots = P.nvals;
-    g->info.n_levels = P.nlev;
-    g->info.n_back_levels = P.nblev;
-    g->info.n_pairs = (int64_t)P.pairs.size() / 4;
-    g->info.flops = P.flops;
-    g->yr_ptr.upload(P.yr_ptr); g->yr_col.upload(P.yr_col); g->yr_pos.upload(P.yr_pos);
-    {
-        std::vector<int> pc(2 * P.yr_pos.size());
-        for (size_t k = 0; k < P.yr_pos.size(); ++k) { pc[2 * k] = P.yr_pos[k]; pc[2 * k + 1] = P.yr_col[k]; }
-        g->yr_pc.upload(pc.empty() ? std::vector<int>(2, 0) : pc);
-        // column-major row table, width the longest row rounded up to kEll columns
-        const int n = (int)P.yr_ptr.size() - 1;
-        int w = 1;
-        for (int r = 0; r < n; ++r) w = std::max(w, P.yr_ptr[r + 1] - P.yr_ptr[r]);
-        w = (w + kEll - 1) / kEll * kEll;
-        g->ell_w = w;
-        std::vector<int> ell(2 * (size_t)w * std::max(n, 1), 0);
-        for (int r = 0; r < n; ++r)
-            for (int k = 0; k < w; ++k) {
-                const int q = P.yr_ptr[r] + k;
-                const bool in = q < P.yr_ptr[r + 1];
-                ell[2 * ((size_t)k * n + r)] = in ? P.yr_pos[q] : -1;
-                ell[2 * ((size_t)k * n + r) + 1] = in ? P.yr_col[q] : r;
-            }
-        g->yr_ell.upload(ell);
+    if (rows) {
+        g->info.n_bus = g->Y.n;
+        g->info.n_jac = P.N;
+        g->info.nnz_ybus = P.nnzY;
+        g->info.nnz_jac = P.nJ;
+        g->info.nnz_lu = P.nnzLU;
+        g->info.n_slots = P.nvals;
+        g->info.n_levels = P.nlev;
+        g->info.n_back_levels = P.nblev;
+        g->info.n_pairs = (int64_t)P.pairs.size() / 4;
+        g->info.flops = P.flops;
+        upload_rows(g);
     }
     auto up_or = [](auto& d, const auto& v, size_t minsz) {
         auto w = v;
@@ -2767,7 +2720,17 @@ void build_plan(pfgpu_grid* g, const std::vector<int>* perm) {
     g->j_ypos.upload(P.j_ypos); g->j_rbus.upload(P.j_rbus); g->j_cbus.upload(P.j_cbus); g->j_sel.upload(P.j_sel);
     g->j_cval.upload(P.j_cval); g->j_slot.upload(P.j_slot);
     g->zero_slots.upload(P.zero_slots.empty() ? std::vector<int>(1, 0) : P.zero_slots);
-    g->w.upload(g->w_h);
+    g->scalar_plan = true;
+}
+
+void build_plan(pfgpu_grid* g, const std::vector<int>* perm) {
+    if (!g->dc && pfgpu::has_block_form(g->J)) build_blocks(g);
+    if (!g->blk) build_scalar(g, perm, true);
+}
+
+// The scalar plan of a grid whose solves run on the block plan.
+void ensure_scalar_plan(pfgpu_grid* g) {
+    if (!g->scalar_plan) build_scalar(g, nullptr, false);
 }
 
 // The J entries of a fast-decoupled grid become constants: B'(row bus, column bus) on the P-row /
@@ -2930,8 +2893,10 @@ int pfgpu_autotune_device(pfgpu_ctx* ctx, pfgpu_grid* grid, int ninst, const dou
         pfgpu_grid* pg = grid->alt_active ? grid->alt.get() : grid;  // the plan in use
         for (int G = 1; G <= kMaxG; G <<= 1) {
             for (int NT : {256, 1024}) {
-                LaunchChoice lc = choose_launch(ctx, pg->P, ninst, fsize, G, NT);
-                if (lc.G != G) continue;  // the dense tail did not fit at this G
+                // the dense tail did not fit at this G
+                if ((pg->blk ? choose_block(ctx, *pg->blk, ninst, fsize, G, NT).G
+                             : choose_launch(ctx, pg->P, ninst, fsize, G, NT).G) != G)
+                    continue;
                 q.G_req = G;
                 q.NT_req = NT;
                 double tmin = 1e300;
