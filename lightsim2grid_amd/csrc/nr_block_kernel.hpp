@@ -180,19 +180,25 @@ __device__ __forceinline__ void tail_sweep(LP T, int m, Put put) {
 }
 
 // v of the lane D lanes below (a sum towards the higher lanes: their last lane is the team's leader).
-// Below 16: within rows of 16 lanes, by DPP; lanes whose source lies outside the row get 0.
-template <int D>
+// Below 16: within rows of 16 lanes, by DPP; lanes whose source lies outside the row get 0. With LAST, in steps
+// of 16 and 32 every lane gets the value of the last lane of the row (of the 32 lanes) below instead, which is
+// the leader's own addend: row_bcast:15 and row_bcast:31.
+template <int D, bool LAST>
+constexpr int kDppBelow = D < 16 ? 0x110 + D : !LAST ? 0 : D == 16 ? 0x142 : 0x143;
+template <int D, bool LAST>
 __device__ __forceinline__ float from_below(float v) {
     const int x = __builtin_bit_cast(int, v);
-    if constexpr (D < 16) return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, x, 0x110 + D, 0xf, 0xf, true));
+    constexpr int dpp = kDppBelow<D, LAST>;
+    if constexpr (dpp) return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, x, dpp, 0xf, 0xf, true));
     else return __shfl_up(v, D);
 }
-template <int D>
+template <int D, bool LAST>
 __device__ __forceinline__ double from_below(double v) {
-    if constexpr (D < 16) {
+    constexpr int dpp = kDppBelow<D, LAST>;
+    if constexpr (dpp) {
         const long long b = __builtin_bit_cast(long long, v);
-        const int lo = __builtin_amdgcn_update_dpp(0, (int)(b & 0xffffffffLL), 0x110 + D, 0xf, 0xf, true);
-        const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0x110 + D, 0xf, 0xf, true);
+        const int lo = __builtin_amdgcn_update_dpp(0, (int)(b & 0xffffffffLL), dpp, 0xf, 0xf, true);
+        const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), dpp, 0xf, 0xf, true);
         return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned int)lo);
     } else {
         return __shfl_up(v, D);
@@ -203,7 +209,7 @@ template <int G, int N, typename FT>
 __device__ __forceinline__ void team_last(FT (&v)[N], int lt) {
     auto add = [&](auto d) {
 #pragma unroll
-        for (int i = 0; i < N; ++i) v[i] += from_below<decltype(d)::value>(v[i]);
+        for (int i = 0; i < N; ++i) v[i] += from_below<decltype(d)::value, G == 1>(v[i]);
     };
     if (lt > 0) {
         add(std::integral_constant<int, G>{});
@@ -658,18 +664,52 @@ __global__ void __launch_bounds__(NT) k_nr_block(const BArgs a) {
         p0 = p[0];
         p1 = p[G];
     };
-    auto any2 = [&](int off, ft2& p0, ft2& p1) {
-        if (off < lds_end) {
-            lds2(off, p0, p1);
-        } else {
-            const ft2* const p = (const ft2*)((const char*)Pg + (size_t)(unsigned)(off - lds_end)) + g;
-            p0 = p[0];
-            p1 = p[G];
+    auto lds1 = [&](int off) -> ft2 { return *(lds_ft2*)(size_t)(unsigned)(off + xg); };
+    // N blocks by offset, from anywhere if `far`: then every lane reads both LDS and memory (its first pair,
+    // where the other is wanted) and selects, all reads issued before the first is waited for. As branches,
+    // the reads of both sides fill the same registers and the compiler waits for each before it issues the
+    // next: three or four memory latencies in turn per unit instead of one (factor levels of the 10 000-bus
+    // N-1 in FP32 9.1 -> 7.6 ms per workgroup, of the 2000-bus one in FP64 2.17 -> 1.9 ms).
+    auto fetch = [&](bool far, const auto& off, auto& p) {
+        constexpr int N = sizeof(p) / sizeof(p[0]);
+        if (!far) {
+#pragma unroll
+            for (int i = 0; i < N; ++i) lds2(off[i], p[i][0], p[i][1]);
+            return;
         }
+        ft2 f[N][2];
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const ft2* const q = (const ft2*)((const char*)Pg + (size_t)(unsigned)max(off[i] - lds_end, 0)) + g;
+            f[i][0] = q[0];
+            f[i][1] = q[G];
+        }
+#pragma unroll
+        for (int i = 0; i < N; ++i) lds2(off[i] < lds_end ? off[i] : 0, p[i][0], p[i][1]);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                p[i][h].x = off[i] < lds_end ? p[i][h].x : f[i][h].x;
+                p[i][h].y = off[i] < lds_end ? p[i][h].y : f[i][h].y;
+            }
     };
-    auto any1 = [&](int off) -> ft2 {
-        if (LEAN || off < lds_end) return *(lds_ft2*)(size_t)(unsigned)(off + xg);
-        return ((const ft2*)((const char*)Pg + (size_t)(unsigned)(off - lds_end)))[g];
+    // the same of N single pairs
+    auto fetch1 = [&](const auto& off, auto& p) {
+        constexpr int N = sizeof(p) / sizeof(p[0]);
+        ft2 f[N];
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+            f[i] = ((const ft2*)((const char*)Pg + (size_t)(unsigned)max(off[i] - lds_end, 0)))[g];
+#pragma unroll
+        for (int i = 0; i < N; ++i) p[i] = lds1(off[i] < lds_end ? off[i] : 0);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            p[i].x = off[i] < lds_end ? p[i].x : f[i].x;
+            p[i].y = off[i] < lds_end ? p[i].y : f[i].y;
+        }
     };
     bool bad = false;   // a zero or non-finite pivot met by this lane
     bool grow = false;  // a pivot that lost more than growth_tau of its value to cancellation
@@ -805,19 +845,8 @@ __global__ void __launch_bounds__(NT) k_nr_block(const BArgs a) {
             walk_levels(next, a.f_mask + (size_t)wave * a.f_words, a.nlev, [&](int4& q) -> bool {
                 const int w = copy_of(q.w), wu = __builtin_amdgcn_readfirstlane(w);
                 const bool far = !LEAN && wu < 0;  // an operand of the wave lies outside LDS
-                ft2 l0, l1, u0, u1, d0, d1;
-                if (far) {
-                    any2(q.x, l0, l1);
-                    any2(q.y, u0, u1);
-                    any2(q.z, d0, d1);
-                } else {
-                    lds2(q.x, l0, l1);
-                    lds2(q.y, u0, u1);
-                    lds2(q.z, d0, d1);
-                }
-                q = *next;
-                next += 64;
-                auto product = [&]() {
+                auto product = [&](const auto& p) {
+                    const ft2 l0 = p[0][0], l1 = p[0][1], u0 = p[1][0], u1 = p[1][1], d0 = p[2][0], d1 = p[2][1];
                     const FT t00 = l0.x * d0.x + l0.y * d1.x, t01 = l0.x * d0.y + l0.y * d1.y;
                     const FT t10 = l1.x * d0.x + l1.y * d1.x, t11 = l1.x * d0.y + l1.y * d1.y;
                     c[0] = fma(t01, u0.y, fma(t00, u0.x, c[0]));
@@ -825,16 +854,39 @@ __global__ void __launch_bounds__(NT) k_nr_block(const BArgs a) {
                     c[2] = fma(t11, u0.y, fma(t10, u0.x, c[2]));
                     c[3] = fma(t11, u1.y, fma(t10, u1.x, c[3]));
                 };
-                if (!(wu & kBlkEnd)) {
-                    product();
-                    return false;
-                }
+                auto ahead = [&]() {
+                    q = *next;
+                    next += 64;
+                };
+                const bool end = wu & kBlkEnd;
                 // the task's last unit: its target's old value is read along
-                const int to = (w & kBlkAssign) ? a.zpair * kPair : (w & kBlkAddrMask) * kPair;
-                ft2 p0, p1;
-                if (far) any2(to, p0, p1);
-                else lds2(to, p0, p1);
-                product();
+                auto target = [&]() { return (w & kBlkAssign) ? a.zpair * kPair : (w & kBlkAddrMask) * kPair; };
+                ft2 p[4][2];
+                if constexpr (LEAN) {
+                    lds2(q.x, p[0][0], p[0][1]);
+                    lds2(q.y, p[1][0], p[1][1]);
+                    lds2(q.z, p[2][0], p[2][1]);
+                    ahead();
+                    if (!end) {
+                        product(p);
+                        return false;
+                    }
+                    lds2(target(), p[3][0], p[3][1]);
+                    product(p);
+                } else if (!end) {
+                    const int off[3] = {q.x, q.y, q.z};
+                    ft2 o[3][2];
+                    fetch(far, off, o);
+                    ahead();
+                    product(o);
+                    return false;
+                } else {
+                    const int off[4] = {q.x, q.y, q.z, target()};
+                    fetch(far, off, p);
+                    ahead();
+                    product(p);
+                }
+                const ft2 p0 = p[3][0], p1 = p[3][1];
                 team_last<G>(c, (wu >> kBlkTeamShift) & 7);
                 if (w & kBlkLead) X.put(w, p0, p1, c[0], c[1], c[2], c[3], false, gtau, bad, grow);
                 c[0] = c[1] = c[2] = c[3] = (FT)0;
@@ -897,26 +949,44 @@ __global__ void __launch_bounds__(NT) k_nr_block(const BArgs a) {
             const int4* next = b_units;
             walk_levels(next, a.b_mask + (size_t)wave * a.b_words, a.nblev, [&](int4& q) -> bool {
                 const int w = copy_of(q.w), wu = __builtin_amdgcn_readfirstlane(w), d = copy_of(q.z);
-                ft2 u0, u1;
-                if constexpr (LEAN) lds2(q.x, u0, u1);
-                else any2(q.x, u0, u1);
-                const ft2 x = any1(q.y);
-                q = *next;
-                next += 64;
-                auto product = [&]() {
+                auto product = [&](const ft2 u0, const ft2 u1, const ft2 x) {
                     const FT v0 = w < 0 ? u1.x : (FT)0, v1 = w < 0 ? u1.y : (FT)0;  // else not the block's
                     c[0] = fma(v0, x.y, fma(u0.x, x.x, c[0]));
                     c[1] = fma(v1, x.y, fma(u0.y, x.x, c[1]));
                 };
-                if (!(wu & kBlkEnd)) {
-                    product();
+                auto ahead = [&]() {
+                    q = *next;
+                    next += 64;
+                };
+                constexpr int kNext = kPair;  // a block's second pair
+                const bool end = wu & kBlkEnd;
+                const int to = (w & kBlkAddrMask) * kPair;
+                ft2 p[6];
+                if constexpr (LEAN) {
+                    lds2(q.x, p[0], p[1]);
+                    p[2] = lds1(q.y);
+                    ahead();
+                    if (!end) {
+                        product(p[0], p[1], p[2]);
+                        return false;
+                    }
+                    lds2(d, p[3], p[4]);
+                    p[5] = lds1(to);
+                    product(p[0], p[1], p[2]);
+                } else if (!end) {
+                    const int off[3] = {q.x, q.x + kNext, q.y};
+                    ft2 o[3];
+                    fetch1(off, o);
+                    ahead();
+                    product(o[0], o[1], o[2]);
                     return false;
+                } else {
+                    const int off[6] = {q.x, q.x + kNext, q.y, d, d + kNext, to};
+                    fetch1(off, p);
+                    ahead();
+                    product(p[0], p[1], p[2]);
                 }
-                ft2 d0, d1;
-                if constexpr (LEAN) lds2(d, d0, d1);
-                else any2(d, d0, d1);
-                const ft2 y = any1((w & kBlkAddrMask) * kPair);
-                product();
+                const ft2 d0 = p[3], d1 = p[4], y = p[5];
                 team_last<G>(c, (wu >> kBlkTeamShift) & 7);
                 if (w & kBlkLead) {
                     const FT v0 = y.x - c[0], v1 = y.y - c[1];
