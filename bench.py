@@ -375,8 +375,8 @@ def large_grid_run(with_cpu: bool, nthreads: int, n_out: int = 5000, n_snap: int
                    "achieved_gbs": algorithmic_bytes(info, iters[status == 0], w) / st["kernel_s"] / 1e9,
                    "hbm_frac": algorithmic_bytes(info, iters[status == 0], w) / st["kernel_s"] / 1e9 / HBM_PEAK_GBS,
                    "flop_rate": flop_rate(info, iters[status == 0], st["kernel_s"], w)}
-        # one solve: the default launch (a wide launch: every workgroup on the one instance, level
-        # by level) and the batched kernel's one workgroup per instance
+        # one solve: the default launch (the one for a single instance's shortest time) and one
+        # workgroup per instance asked for
         one = (dptr[:2], dpos[:dptr[1]], dval[:dptr[1]])
         for G, key in ((0, "single_solve_kernel_ms"), (1, "single_solve_one_workgroup_kernel_ms")):
             lat = []
@@ -530,8 +530,8 @@ def dc_fdpf_run(with_cpu: bool, reps: int = 20) -> dict:
 
 
 def single_solves(name: str, reps: int = 5) -> dict:
-    """One solve of a synthetic grid from its V0, reps times per form: the default launch (a wide
-    launch, every workgroup on the one instance, for a large plan) and one workgroup per instance."""
+    """One solve of a synthetic grid from its V0, reps times per form: the default launch (the one for a
+    single instance's shortest time, on a large plan) and one workgroup per instance asked for."""
     from lightsim2grid_amd import abi, gridgen
     g = gridgen.make(name)
     d = g.solver_inputs()

@@ -1348,8 +1348,7 @@ struct pfgpu_grid {
     };
     std::vector<std::unique_ptr<Streams>> streams;  // by (G, block size, value size, lean)
     // Block form of the factorisation (blocks.hpp), the plan of every AC and fast-decoupled solve on
-    // J's own diagonal; the scalar plan P then holds only the sizes and Ybus rows until a launch needs
-    // it (ensure_scalar_plan: wide launches)
+    // J's own diagonal; the scalar plan P then holds only the sizes and Ybus rows
     struct Block {
         pfgpu::BlockPlan P;
         DevBuf<int> bus_y, tail_src, rows, jd_ptr, jd, jd_pos, jd_jidx, row_jidx, y_row, y_ent, jc_dst, jc_jidx;
@@ -1362,7 +1361,6 @@ struct pfgpu_grid {
         std::map<int, std::unique_ptr<Lanes>> lanes;  // by (G, block size, value size)
     };
     std::unique_ptr<Block> blk, blk_life;  // value pairs by use; by life, for launches that overlay V (build_blocks)
-    bool scalar_plan = false;
     // autotuned launch shape per precision (G, block), 0 = not tuned
     int tuned_G[2] = {0, 0}, tuned_NT[2] = {0, 0};
     // the next solve's first iteration is the solver's first factorisation (KLULinearSolver::
@@ -1685,10 +1683,10 @@ struct FixedScratch {
     size_t ws_bytes = 0;
 };
 
-// Wide launches: one instance at a time over every workgroup of the device (wide.hpp). Taken for
-// instances_per_wg == -1, and by default for a single launch unit (one instance, or one chain of
-// time steps) on a plan of at least kWidePairs factor pairs, where one workgroup per instance would
-// leave the device idle. Not for DC grids, J captures or the allocation-free entry point.
+// Launches for the shortest time of one instance. Taken for instances_per_wg == -1, and by default for a
+// single launch unit (one instance, or one chain of time steps) on a plan of at least kWidePairs factor
+// pairs. Not for DC grids, J captures or the allocation-free entry point. On a plan without a block form
+// they are wide: one instance at a time over every workgroup of the launch (wide.hpp).
 constexpr long long kWidePairs = 200000;
 constexpr int kWideBlocks = 32;  // workgroups of a wide launch (PFGPU_WIDE_BLOCKS overrides)
 
@@ -1713,11 +1711,8 @@ std::vector<int> level_teams(const std::vector<int>& lvl, const std::vector<int>
     return out;
 }
 
-void ensure_scalar_plan(pfgpu_grid* g);
-
 void launch_wide(pfgpu_ctx* ctx, pfgpu_grid* gr, const SolveArgs& q, int precision, int nunits, const int* imap,
                  const AuxLayout& AL, bool fresh, pfgpu_stats* st) {
-    ensure_scalar_plan(gr);
     const pfgpu::DevicePlan& P = gr->P;
     const int n = P.n;
     const bool fp32 = precision != PFGPU_FP64;
@@ -2084,14 +2079,23 @@ void launch_pass(pfgpu_ctx* ctx, pfgpu_grid* gr, const SolveArgs& q, int precisi
                  int nunits, const int* imap, const AuxLayout& AL, bool fresh, pfgpu_stats* st,
                  const FixedScratch* fx = nullptr) {
     if (wide_wanted(gr, q, G_req, nunits, fx)) {
-        launch_wide(ctx, gr, q, precision, nunits, imap, AL, fresh, st);
+        // A plan with a block form takes one workgroup per instance here too: the grid-wide barrier of every
+        // level costs more than the other workgroups' lanes give. One solve from V0 in FP64 (FP32), ms:
+        // 2000 buses 0.68 against 2.3 wide, 5000 1.3 (0.9) against 3.4, 10 000 3.9 (2.8) against 8.2 (7.7),
+        // 20 000 9.8 (7.3) against 25 (22), 40 000 24 (18) against 51 (45).
+        if (gr->blk) {
+            launch_block(ctx, gr, q, precision, 1, 1024, nunits, imap, AL, fresh, st, fx);
+            if (st) st->instances_per_wg = -1;
+        } else {
+            launch_wide(ctx, gr, q, precision, nunits, imap, AL, fresh, st);
+        }
         return;
     }
     const pfgpu::DevicePlan& P = gr->P;
     const int n = P.n;
     const int fsize = precision == PFGPU_FP64 ? 8 : 4;
     const int pslot = precision == PFGPU_FP64 ? 0 : 1;
-    if (G_req == -1) G_req = 0;  // a wide launch was not possible here (DC grid, J capture, fixed scratch)
+    if (G_req == -1) G_req = 0;  // not here (DC grid, J capture, fixed scratch)
     if (G_req == 0 && NT_req == 0 && gr->tuned_G[pslot]) {
         G_req = gr->tuned_G[pslot];
         NT_req = gr->tuned_NT[pslot];
@@ -2681,24 +2685,22 @@ void build_blocks(pfgpu_grid* g) {
     g->info.flops = fc.flops;
 }
 
-void build_scalar(pfgpu_grid* g, const std::vector<int>* perm, bool rows) {
+void build_scalar(pfgpu_grid* g, const std::vector<int>* perm) {
     pfgpu::SymbolicLU S = pfgpu::symbolic_lu(g->J, 96, perm);
     pfgpu::Schedule sch = pfgpu::build_schedule(S);
     g->P = pfgpu::build_device_plan(g->Y, g->J, S, sch);
     const auto& P = g->P;
-    if (rows) {
-        g->info.n_bus = g->Y.n;
-        g->info.n_jac = P.N;
-        g->info.nnz_ybus = P.nnzY;
-        g->info.nnz_jac = P.nJ;
-        g->info.nnz_lu = P.nnzLU;
-        g->info.n_slots = P.nvals;
-        g->info.n_levels = P.nlev;
-        g->info.n_back_levels = P.nblev;
-        g->info.n_pairs = (int64_t)P.pairs.size() / 4;
-        g->info.flops = P.flops;
-        upload_rows(g);
-    }
+    g->info.n_bus = g->Y.n;
+    g->info.n_jac = P.N;
+    g->info.nnz_ybus = P.nnzY;
+    g->info.nnz_jac = P.nJ;
+    g->info.nnz_lu = P.nnzLU;
+    g->info.n_slots = P.nvals;
+    g->info.n_levels = P.nlev;
+    g->info.n_back_levels = P.nblev;
+    g->info.n_pairs = (int64_t)P.pairs.size() / 4;
+    g->info.flops = P.flops;
+    upload_rows(g);
     auto up_or = [](auto& d, const auto& v, size_t minsz) {
         auto w = v;
         if (w.size() < minsz) w.resize(minsz);
@@ -2720,17 +2722,11 @@ void build_scalar(pfgpu_grid* g, const std::vector<int>* perm, bool rows) {
     g->j_ypos.upload(P.j_ypos); g->j_rbus.upload(P.j_rbus); g->j_cbus.upload(P.j_cbus); g->j_sel.upload(P.j_sel);
     g->j_cval.upload(P.j_cval); g->j_slot.upload(P.j_slot);
     g->zero_slots.upload(P.zero_slots.empty() ? std::vector<int>(1, 0) : P.zero_slots);
-    g->scalar_plan = true;
 }
 
 void build_plan(pfgpu_grid* g, const std::vector<int>* perm) {
     if (!g->dc && pfgpu::has_block_form(g->J)) build_blocks(g);
-    if (!g->blk) build_scalar(g, perm, true);
-}
-
-// The scalar plan of a grid whose solves run on the block plan.
-void ensure_scalar_plan(pfgpu_grid* g) {
-    if (!g->scalar_plan) build_scalar(g, nullptr, false);
+    if (!g->blk) build_scalar(g, perm);
 }
 
 // The J entries of a fast-decoupled grid become constants: B'(row bus, column bus) on the P-row /

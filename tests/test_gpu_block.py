@@ -79,3 +79,35 @@ def test_block_kernel_where_v_and_values_lie(gpu_ctx, oracle_mod, n, prec):
     rng = np.random.default_rng(n)
     conts = [[int(k)] for k in rng.choice(g.nbr, 5, replace=False)]
     _check(oracle_mod, gpu_ctx, g, conts, prec, 1)
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+def test_shortest_time_launch_with_and_without_a_block_form(gpu_ctx, oracle_mod, prec):
+    """instances_per_wg = -1: on the block plan bit-equal to one workgroup of 1024 lanes per instance; on the plan
+    of a re-pivoted grid, which has no block form, the wide kernel, equal to the oracle."""
+    from conftest import zero_diagonal_grid
+    from lightsim2grid_amd import abi
+    _say("shortest time", prec)
+    g = _grid(900, 1.5, 3, 0.3)
+    d = g.solver_inputs()
+    gr = abi.Grid(gpu_ctx, d["Ybus"], d["slack_ids"], d["slack_weights"], d["pv"], d["pq"])
+    a = (gr.ybus_values(d["Ybus"]), d["Sbus"], d["V0"], 10, 1e-8)
+    r = gr.solve(*a, precision=prec, instances_per_wg=-1)
+    gr.reset()
+    r1 = gr.solve(*a, precision=prec, instances_per_wg=1)
+    assert r["stats"]["instances_per_wg"] == -1 and r1["stats"]["instances_per_wg"] == 1
+    assert r["status"][0] == 0 and np.max(np.abs(r["V"] - r1["V"])) <= (1e-9 if prec == abi.FP64 else 5e-8)
+    if r1["stats"]["block_size"] == r["stats"]["block_size"]:
+        assert np.array_equal(r["V"], r1["V"])
+
+    d = zero_diagonal_grid()
+    o = oracle_mod.OracleNR(False)
+    assert o.compute_pf(d["Ybus"], d["V0"], d["Sbus"], d["slack_ids"], d["slack_weights"], d["pv"], d["pq"], 10, 1e-8)
+    gr = abi.Grid(gpu_ctx, d["Ybus"], d["slack_ids"], d["slack_weights"], d["pv"], d["pq"])
+    Yx = gr.ybus_values(d["Ybus"])
+    for _ in range(2):  # the plan is kept: the second solve runs on it alone
+        r = gr.solve(Yx, d["Sbus"], d["V0"], 10, 1e-8, precision=prec, instances_per_wg=-1)
+        assert r["stats"]["instances_per_wg"] == -1
+        assert r["status"][0] == 0 and r["iters"][0] == o.get_nb_iter()
+        assert np.max(np.abs(r["V"][0] - o.get_V())) <= 1e-8
+    assert r["stats"]["workgroups"] > 1  # the wide kernel's
