@@ -74,9 +74,8 @@ Arms symbolic(int nb, std::vector<std::vector<int>>& low) {
     return A;
 }
 
-// Unknowns of the dense tail at most (its tile is kept in LDS and factored by one workgroup), and
-// the smallest tail worth a dense phase of its own.
-constexpr int kMaxTail = 96, kMinTail = 8;
+// The smallest tail worth a dense phase of its own.
+constexpr int kMinTail = 8;
 
 }  // namespace
 
@@ -163,10 +162,9 @@ BlockPlan build_block_plan(const YbusPattern& Y, const JPattern& J, const std::v
         P.nblev = std::max(P.nblev, l + 1);
     }
 
-    // --- storage: tile, zero pairs, right-hand sides / solutions, then the recycled blocks --------
-    P.tile_pairs = (m * (m + 1) + 1) / 2;
-    P.zpair = P.tile_pairs;
-    int next = P.tile_pairs + 2;
+    // --- storage: zero pairs, then the recycled blocks and the right-hand sides / solutions ----------
+    P.zpair = 0;
+    int next = 2;
     std::vector<int> addr(nv, -1);
     struct Life { int id, t0, t1; long long acc; };
     std::vector<Life> one, two, rhs;
@@ -209,7 +207,11 @@ BlockPlan build_block_plan(const YbusPattern& Y, const JPattern& J, const std::v
     // a block takes the place of one that was read for the last time before it is written (interval
     // colouring by size); places by decreasing accesses, so that a launch that cannot hold all of
     // them in LDS keeps the most used
-    struct Place { int size; long long acc; bool fill; std::vector<int> ids; };  // fill: empty during the assembly
+    struct Place { int size; long long acc; bool fill, tail; std::vector<int> ids; };  // fill: empty during the assembly
+    auto in_tail = [&](int id) {
+        if (id < 2 * nb) return id % nb >= k0;
+        return (id < vU ? id - vL : id - vU) >= A.cp[k0];
+    };
     std::vector<Place> places;
     auto colour = [&](std::vector<Life>& v, int size) {
         std::stable_sort(v.begin(), v.end(), [](const Life& a, const Life& b) { return a.t0 < b.t0; });
@@ -222,10 +224,11 @@ BlockPlan build_block_plan(const YbusPattern& Y, const JPattern& J, const std::v
                 free.pop();
             } else {
                 p = (int)places.size();
-                places.push_back({size, 0, true, {}});
+                places.push_back({size, 0, true, false, {}});
             }
             places[p].ids.push_back(x.id);
             places[p].acc += x.acc;
+            places[p].tail |= in_tail(x.id);
             if (x.t0 <= 0 || x.id >= nb && x.id < vL) places[p].fill = false;
             free.push({x.t1, p});
         }
@@ -237,6 +240,7 @@ BlockPlan build_block_plan(const YbusPattern& Y, const JPattern& J, const std::v
     std::iota(po.begin(), po.end(), 0);
     std::stable_sort(po.begin(), po.end(), [&](int a, int b) {
         if (order == kByLife && places[a].fill != places[b].fill) return places[b].fill;
+        if (order == kByUse && places[a].tail != places[b].tail) return places[a].tail;
         return places[a].acc * places[b].size > places[b].acc * places[a].size;
     });
     P.second.assign(next, 0);
@@ -245,6 +249,7 @@ BlockPlan build_block_plan(const YbusPattern& Y, const JPattern& J, const std::v
         if (order == kByLife && places[p].fill && P.fill_at < 0) P.fill_at = next;
         for (int id : places[p].ids) addr[id] = next;
         next += places[p].size;
+        if (places[p].tail) P.fixed_pairs = next;
         P.second.push_back(0);
         if (places[p].size == 2) P.second.push_back(1);
     }

@@ -11,7 +11,7 @@
 // pair per column of bus j: (U(0, c), U(1, c)) over the rows of bus k. The inner dimension is always
 // padded to 2 with zeros, so a product L D U needs no test of a block's size. A diagonal block takes
 // two row pairs and ends as the inverse of its pivot block; a right-hand side / solution entry of a bus
-// is one pair. The tail of the elimination order is a dense scalar tile.
+// is one pair. The tail of the elimination order is factored as one dense matrix.
 #pragma once
 
 #include <cstdint>
@@ -37,11 +37,15 @@ constexpr int kBlkLevel = 1 << 30;                 // last unit of the wave's le
 constexpr int kBlkWide = (int)(1u << 31);          // the block of U has two columns (backward); an operand of the
                                                    // wave lies outside LDS (factor)
 
+// Unknowns of the dense tail at most: a wave factors it in registers, a column to a register and a row to
+// a lane (nr_block_kernel.hpp), which at 1024 lanes leaves room for 48 columns of FP64. (The 10 000-bus grid's top chain has 88 unknowns: the
+// 40 below the tail take 20 levels more, as long as the 40 took in a tail of 16 waves.)
+constexpr int kMaxTail = 48;
+
 struct BlockPlan {
     int n = 0, m = 0;        // buses, unknowns of the dense tail
-    int tile_pairs = 0;      // pairs [0, tile_pairs) are the dense phase's tile: scalars, row-major, row
-                             // stride m + 1, the right-hand side as column m
-    int zpair = 0;           // two pairs that always hold zeros (tile_pairs, tile_pairs + 1)
+    int zpair = 0;           // two pairs that always hold zeros (0 and 1)
+    int fixed_pairs = 2;     // the pairs below lie in LDS in every launch: the zeros, the tail's places
     int npairs = 0;          // value pairs of one instance, one pad pair at the end included
     int nlev = 0, nblev = 0;
     // per bus: the pair of its right-hand side (P, Q) and solution (dVa, dVm), kBlkIn2: two of them;
@@ -49,7 +53,7 @@ struct BlockPlan {
     // slack's bus), -1 without one
     std::vector<int> bus_y;
     int slack_x = -1, slack_bus = -1;
-    // where the dense phase finds its tile: per entry, row-major [m][m + 1], the number's place (2 pair +
+    // where the dense phase finds its matrix: per entry, row-major [m][m + 1], the number's place (2 pair +
     // component); column m is the right-hand side, which receives the solution
     std::vector<int> tail_src;
     std::vector<char> second;   // per pair: the second one of a block (npairs + 1 entries)

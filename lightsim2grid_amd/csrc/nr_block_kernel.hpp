@@ -46,137 +46,83 @@ using pfgpu_block::BArgs;
 
 static_assert(kMaxEdits == pfgpu_block::kEdits);
 
-// ---------------------------------------------------------------------------
-// Dense tail with one instance per workgroup: the tile's rows in registers, two at a time to a wave in
-// turn, lane = column. Step p eliminates rows 2p, 2p + 1: their wave factors the 2 x 2 pivot and writes
-// the two rows of U (reciprocal pivots on the diagonal) to the tile; behind the barrier every wave takes
-// its factors of L from its own rows by lane reads and updates them, the owner of the next rows first.
-// ---------------------------------------------------------------------------
-// Out of line, as the other phases that hold many values: inlined, its registers and the walks' add up
-// to spills in both (128 VGPRs at 1024 lanes). Returns whether a pivot was zero or non-finite.
-// src: where the factor levels left the tile's numbers (row-major, m + 1 columns): below 2 nlds in LDS.
-template <typename FT, int NW, int MAXP, int CS, typename LP>
-__device__ __noinline__ bool tail_registers(LP T, int m_, const int* src, const FT* spill, int nlds2) {
-    const int m = __builtin_amdgcn_readfirstlane(m_);
-    bool bad = false;
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), ld = m + 1;
-    FT R[MAXP][2][CS];
-#pragma unroll
-    for (int a = 0; a < MAXP; ++a)
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-            for (int c = 0; c < CS; ++c) {
-                const int x = src[min(2 * (a * NW + wave) + h, m - 1) * ld + min(lane + 64 * c, m)];
-                if (x < nlds2) R[a][h][c] = T[x];
-                else R[a][h][c] = spill[x - nlds2];
-            }
-    // column k (uniform) of a row
-    auto at = [&](const FT (&r)[CS], int k) -> FT {
-        if constexpr (CS == 1) return lane_read(r[0], k);
-        else return lane_read(k < 64 ? r[0] : r[1], k & 63);
-    };
-    auto publish = [&](FT (&q)[2][CS], int k) {
-        const FT d0 = at(q[0], k);
-        bad |= bad_pivot(d0);
-        const FT r0 = pivot_recip(d0);
-        const bool two = k + 1 < m;
-        FT r1 = (FT)0;
-        if (two) {
-            const FT l = at(q[1], k) * r0;
-#pragma unroll
-            for (int c = 0; c < CS; ++c) q[1][c] -= l * q[0][c];
-            const FT d1 = at(q[1], k + 1);
-            bad |= bad_pivot(d1);
-            r1 = pivot_recip(d1);
-        }
-#pragma unroll
-        for (int c = 0; c < CS; ++c) {
-            const int j = lane + 64 * c;
-            if (j >= k && j <= m) T[k * ld + j] = j == k ? r0 : q[0][c];
-            if (two && j > k && j <= m) T[(k + 1) * ld + j] = j == k + 1 ? r1 : q[1][c];
-        }
-    };
-    if (wave == 0) publish(R[0], 0);
-    __syncthreads();
-#pragma unroll
-    for (int a = 0; a < MAXP; ++a)
-#pragma unroll 1
-        for (int o = 0; o < NW; ++o) {
-            const int k = 2 * (a * NW + o);
-            if (k + 2 >= m) break;
-            FT u0[CS], u1[CS];
-            const FT r0 = T[k * ld + k], r1 = T[(k + 1) * ld + k + 1];
-#pragma unroll
-            for (int c = 0; c < CS; ++c) {
-                u0[c] = T[k * ld + min(lane + 64 * c, m)];
-                u1[c] = T[(k + 1) * ld + min(lane + 64 * c, m)];
-            }
-            auto update = [&](FT (&q)[2][CS]) {
-                const FT l00 = at(q[0], k) * r0, l10 = at(q[1], k) * r0;
-#pragma unroll
-                for (int c = 0; c < CS; ++c) {
-                    q[0][c] -= l00 * u0[c];
-                    q[1][c] -= l10 * u0[c];
-                }
-                const FT l01 = at(q[0], k + 1) * r1, l11 = at(q[1], k + 1) * r1;
-#pragma unroll
-                for (int c = 0; c < CS; ++c) {
-                    q[0][c] -= l01 * u1[c];
-                    q[1][c] -= l11 * u1[c];
-                }
-            };
-            const bool wraps = o + 1 == NW;
-            if (!wraps && wave == o + 1) {
-                update(R[a]);
-                publish(R[a], k + 2);
-            } else if (!wraps && wave > o) {
-                update(R[a]);
-            }
-            if (a + 1 < MAXP) {
-                constexpr int last = MAXP - 1;
-                if (wraps && wave == 0) {
-                    update(R[a + 1 <= last ? a + 1 : last]);
-                    publish(R[a + 1 <= last ? a + 1 : last], k + 2);
-                } else {
-                    update(R[a + 1 <= last ? a + 1 : last]);
-                }
-            }
-#pragma unroll
-            for (int b = a + 2; b < MAXP; ++b) update(R[b]);
-            __syncthreads();
-        }
-    return bad;
+// A pointer that is the same in every lane (one instance per workgroup), in scalar registers.
+template <typename T>
+__device__ __forceinline__ T* uniform(T* p) {
+    const unsigned long long v = (unsigned long long)p;
+    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)v), hi = __builtin_amdgcn_readfirstlane((unsigned)(v >> 32));
+    return (T*)((unsigned long long)hi << 32 | lo);
 }
 
-// The backward sweep of the tail on the first wave, x_k handed on by lane reads: lane s holds rows s and
-// s + 64. put(row, x) stores the solution.
-template <typename FT, typename LP, typename Put>
-__device__ __forceinline__ void tail_sweep(LP T, int m, Put put) {
-    const int s = threadIdx.x, ld = m + 1;
-    FT y0 = s < m ? T[s * ld + m] : (FT)0, y1 = s + 64 < m ? T[(s + 64) * ld + m] : (FT)0;
-    auto col = [&](int k, FT& u0, FT& u1, FT& dk) {
-        const int c = max(k, 0);
-        dk = T[c * ld + c];
-        u0 = T[min(s, m - 1) * ld + c];
-        u1 = T[min(s + 64, m - 1) * ld + c];
-    };
-    FT u0, u1, dk;
-    col(m - 1, u0, u1, dk);
-    for (int k = m - 1; k >= 0; --k) {
-        FT nu0, nu1, ndk;
-        col(k - 1, nu0, nu1, ndk);
-        const FT xk = lane_read(k < 64 ? y0 : y1, k & 63) * dk;
-        if (s == (k & 63)) {
-            if (k < 64) y0 = xk;
-            else y1 = xk;
+// ---------------------------------------------------------------------------
+// Dense tail of one instance on one wave, in registers: lane = row, R[j] = column j, Y = the right-hand side.
+// Rows and columns end at M (tails of m <= M unknowns, preceded by rows and columns of the identity), so that
+// the code is straight: as branches around the missing pivots, the registers meet at joins and are copied
+// there. A pivot row reaches the other lanes by lane reads of each column, the next pivot's column first,
+// whose reciprocal is then formed beside the other columns' updates; no LDS access and no barrier lies
+// between the pivots.
+// src: each number's place, by columns of 64 lanes (2 pair + component; all of them in LDS); the right-hand
+// side's places receive the solution. Returns whether a pivot was zero or non-finite.
+// Bound by the instruction issue of one wave: about M^2 / 2 lane reads and as many updates. 43 unknowns of the
+// 2000-bus grid, per iteration: 8.6 us in FP32, 13.7 in FP64 (two lane reads per value); two rows at a time to
+// one of 16 waves in turn, a barrier and an LDS round trip per pair of pivots, it took 14 and 19 us. With four
+// instances per workgroup (118 buses, 4 waves) each wave takes one: 6 us instead of 15 for all four.
+// Out of line: inlined, its registers and the walks' add up to spills in both.
+// ---------------------------------------------------------------------------
+template <typename FT, int G, int M>
+__device__ __noinline__ bool tail_wave(int m_, int g_, const int* src_) {
+    typedef __attribute__((address_space(3))) FT lds_ft;
+    typedef __attribute__((address_space(1))) const int glb_int;
+    const int m = __builtin_amdgcn_readfirstlane(m_), g = __builtin_amdgcn_readfirstlane(g_);
+    const int lane = threadIdx.x & 63, k0 = M - m;
+    const glb_int* const src = (const glb_int*)uniform((int*)src_) + (pfgpu::kMaxTail - M) + lane;
+    auto at = [&](int x) -> lds_ft* { return (lds_ft*)(size_t)(unsigned)(((2 * G) * (x >> 1) + 2 * g + (x & 1)) * (int)sizeof(FT)); };
+    FT R[M], Y;
+    int from[M];
+#pragma unroll
+    for (int j = 0; j < M; ++j) from[j] = src[max(j - k0, 0) * 64];
+    const int ys = src[m * 64];
+#pragma unroll
+    for (int j = 0; j < M; ++j) R[j] = *at(from[j]);
+    Y = *at(ys);
+#pragma unroll
+    for (int j = 0; j < M; ++j)
+        if (j < M - 8) R[j] = j >= k0 ? R[j] : lane == j ? (FT)1 : (FT)0;
+    bool bad = false;
+    FT D = (FT)0, r = pivot_recip(lane_read(R[0], 0));  // lane k: the reciprocal of pivot k; this pivot's
+#pragma unroll
+    for (int k = 0; k < M; ++k) {
+        bad |= bad_pivot(lane_read(R[k], k));
+        D = lane == k ? r : D;
+        const FT l = lane > k ? R[k] * r : (FT)0;
+        if (k + 1 < M) {
+            R[k + 1] -= l * lane_read(R[k + 1], k);
+            r = pivot_recip(lane_read(R[k + 1], k + 1));
         }
-        if (s < k) y0 -= u0 * xk;  // rows i < k only: a non-finite x_k leaves the others
-        if (s + 64 < k) y1 -= u1 * xk;
-        u0 = nu0; u1 = nu1; dk = ndk;
+        // four lane reads, then four updates: a value just read by lane may not be used at once
+#pragma unroll
+        for (int j = k + 2; j < M; j += 4) {
+            FT u[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (j + i < M) u[i] = lane_read(R[j + i], k);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (j + i < M) R[j + i] -= l * u[i];
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        Y -= l * lane_read(Y, k);
     }
-    if (s < m) put(s, y0);
-    if (s + 64 < m) put(s + 64, y1);
+    FT x = (FT)0;
+#pragma unroll
+    for (int k = M - 1; k >= 0; --k) {
+        const FT xk = lane_read(Y, k) * lane_read(D, k);
+        x = lane == k ? xk : x;
+        Y -= xk * R[k];  // (lanes from k on are done)
+    }
+    if (lane >= k0 && lane < M) *at(ys) = x;
+    return bad;
 }
 
 // v of the lane D lanes below (a sum towards the higher lanes: their last lane is the team's leader).
@@ -308,14 +254,6 @@ struct WgState {
 
 // The kernel's arguments where the launch left them (the phases out of line read them there).
 typedef __attribute__((address_space(4))) const BArgs cargs;
-
-// A pointer that is the same in every lane (one instance per workgroup), in scalar registers.
-template <typename T>
-__device__ __forceinline__ T* uniform(T* p) {
-    const unsigned long long v = (unsigned long long)p;
-    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)v), hi = __builtin_amdgcn_readfirstlane((unsigned)(v >> 32));
-    return (T*)((unsigned long long)hi << 32 | lo);
-}
 
 // One instance's value pairs: the first nlds in LDS, the rest in the workgroup's spill area.
 template <typename FT, int G, bool LEAN>
@@ -622,7 +560,6 @@ __global__ void __launch_bounds__(NT) k_nr_block(const BArgs a) {
     // explicit LDS address space: every access is a ds_read / ds_write
     typedef __attribute__((address_space(3))) FT lds_ft;
     typedef __attribute__((address_space(3))) ft2 lds_ft2;
-    lds_ft* const Xl = (lds_ft*)(lds_raw);    // tile scalars: scalar i of instance g at i * G + g
     lds_ft2* const Pl = (lds_ft2*)(lds_raw);  // pair q of instance g at q * G + g
     const WgState<G> wst((lds_u8*)lds_raw + a.sh_off, NT);
     lds_dbl* const s_part = wst.part;
@@ -898,39 +835,13 @@ __global__ void __launch_bounds__(NT) k_nr_block(const BArgs a) {
         tmark(1);
         // ---- dense tail ---------------------------------------------------------------------------
         if (m > 0) {
-            bool tbad = false;
-            auto get = [&](int i) -> FT {
-                const int x = a.tail_src[i];
-                if (LEAN || (x >> 1) < nlds) return Xl[2 * ((x >> 1) * G + g) + (x & 1)];
-                return reinterpret_cast<const FT*>(Pg + (size_t)((x >> 1) - nlds) * G + g)[x & 1];
-            };
-            auto put_x = [&](int r, FT v) {  // row r of the solution
-                const int x = a.tail_src[r * (m + 1) + m];
-                if (LEAN || (x >> 1) < nlds) Xl[2 * ((x >> 1) * G + g) + (x & 1)] = v;
-                else reinterpret_cast<FT*>(Pg + (size_t)((x >> 1) - nlds) * G + g)[x & 1] = v;
-            };
-            bool swept = false;
-            if constexpr (G == 1 && NT == 1024) {
-                if (m <= 32) tbad = tail_registers<FT, 16, 1, 1>(Xl, m, a.tail_src, (const FT*)Pg, 2 * nlds);
-                else if (m < 64) tbad = tail_registers<FT, 16, 2, 1>(Xl, m, a.tail_src, (const FT*)Pg, 2 * nlds);
-                else tbad = tail_registers<FT, 16, 3, 2>(Xl, m, a.tail_src, (const FT*)Pg, 2 * nlds);
-                swept = true;
-            } else if constexpr (G == 1) {
-                if (m <= 32) {
-                    tbad = tail_registers<FT, 4, 4, 1>(Xl, m, a.tail_src, (const FT*)Pg, 2 * nlds);
-                    swept = true;
-                }
+            for (int gi = wave; gi < G; gi += kWaves) {
+                if (s_done[gi]) continue;
+                const bool tbad = m <= 16   ? tail_wave<FT, G, 16>(m, gi, a.tail_src)
+                                  : m <= 32 ? tail_wave<FT, G, 32>(m, gi, a.tail_src)
+                                            : tail_wave<FT, G, 48>(m, gi, a.tail_src);
+                if (tbad) s_piv[gi] = 1;
             }
-            if (swept) {
-                if (tid < 64) tail_sweep<FT>(Xl, m, put_x);
-            } else {
-                for (int i = s; i < m * (m + 1); i += nslot) Xl[i * G + g] = get(i);
-                __syncthreads();
-                dense_tail_lds<FT, G, NT>(Xl, m, g, s, act, tbad);
-                __syncthreads();
-                for (int r = s; r < m; r += nslot) put_x(r, Xl[(r * (m + 1) + m) * G + g]);
-            }
-            if (tbad) s_piv[g] = 1;
             __syncthreads();
         }
         tmark(2);

@@ -1916,7 +1916,7 @@ BlockChoice choose_block(const pfgpu_ctx* ctx, const pfgpu_grid::Block& b, int n
         return (size_t)ctx->lds_max > fixed ? (size_t)ctx->lds_max - fixed : 0;
     };
     auto values = [&](int G) -> size_t { return (size_t)P.npairs * 2 * G * fsize; };
-    const size_t fixed_pairs = (size_t)P.tile_pairs + 2;  // always in LDS
+    const size_t fixed_pairs = (size_t)P.fixed_pairs;
     BlockChoice c{};
     c.G = 1;
     const long long ncu = std::max(1, ctx->n_cu);
@@ -2647,7 +2647,12 @@ std::unique_ptr<pfgpu_grid::Block> upload_blocks(const pfgpu_grid* g, const std:
         d.upload(v);
     };
     b->bus_y.upload(B.bus_y);
-    up(b->tail_src, B.tail_src);
+    // by columns, a lane per row: rows and columns end at kMaxTail, lanes beside them read a zero (a wave on M
+    // of the columns starts kMaxTail - M lanes into the first, and so ends within one more)
+    std::vector<int> tail(B.m > 0 ? (size_t)(B.m + 2) * 64 : 0, 2 * B.zpair);
+    for (int r = 0; r < B.m; ++r)
+        for (int c = 0; c <= B.m; ++c) tail[(size_t)c * 64 + (pfgpu::kMaxTail - B.m + r)] = B.tail_src[(size_t)r * (B.m + 1) + c];
+    up(b->tail_src, tail);
     b->y_row.upload(g->Y.i);
     const int nrow = (int)B.row_len.size(), nent = (int)B.jd_pos.size();
     std::vector<int> ptr = B.jd_ptr, ent(g->Y.i.size(), -1);

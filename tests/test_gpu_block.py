@@ -1,5 +1,5 @@
 """The block-plan kernel at the edges of its launch shapes and phases, against the oracle: no dense tail, tails
-in one, two and three register row pairs per wave, with one and two columns per lane,
+of each code size of the wave that factors them, tails cut at the largest,
 V beside the values, over them and in memory, values spilled, several instances per workgroup in both block
 sizes, Ybus edits inside and beyond the eight kept in LDS, one and two batches of rows per lane.
 Bar: the FP64 form the oracle's flags and iterations and |V - V_oracle| <= 1e-8; the FP32 form the same flags,
@@ -40,8 +40,8 @@ def _check(oracle_mod, ctx, g, conts, prec, G, block=None):
     return r["stats"]
 
 
-# buses, branches per bus, seed, loading: tails of 0, 8, 17, 30, 38, 51, 84 and 70 unknowns, the last one with
-# 66 levels (two words of the waves' level masks)
+# buses, branches per bus, seed, loading: top chains of 0, 8, 17, 30, 38, 51, 84 and 70 unknowns (the tail takes
+# at most 48 of them), the last one with more than 64 levels (two words of the waves' level masks)
 TAILS = [(6, 1.2, 3, 0.3), (12, 1.3, 1, 0.5), (250, 1.7, 4, 0.2), (400, 1.9, 4, 0.15), (500, 2.4, 6, 0.12),
          (400, 3.3, 1, 0.15), (700, 3.3, 1, 0.12), (1200, 3.3, 2, 0.1)]
 
