@@ -46,85 +46,6 @@ using pfgpu_block::BArgs;
 
 static_assert(kMaxEdits == pfgpu_block::kEdits);
 
-// A pointer that is the same in every lane (one instance per workgroup), in scalar registers.
-template <typename T>
-__device__ __forceinline__ T* uniform(T* p) {
-    const unsigned long long v = (unsigned long long)p;
-    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)v), hi = __builtin_amdgcn_readfirstlane((unsigned)(v >> 32));
-    return (T*)((unsigned long long)hi << 32 | lo);
-}
-
-// ---------------------------------------------------------------------------
-// Dense tail of one instance on one wave, in registers: lane = row, R[j] = column j, Y = the right-hand side.
-// Rows and columns end at M (tails of m <= M unknowns, preceded by rows and columns of the identity), so that
-// the code is straight: as branches around the missing pivots, the registers meet at joins and are copied
-// there. A pivot row reaches the other lanes by lane reads of each column, the next pivot's column first,
-// whose reciprocal is then formed beside the other columns' updates; no LDS access and no barrier lies
-// between the pivots.
-// src: each number's place, by columns of 64 lanes (2 pair + component; all of them in LDS); the right-hand
-// side's places receive the solution. Returns whether a pivot was zero or non-finite.
-// Bound by the instruction issue of one wave: about M^2 / 2 lane reads and as many updates. 43 unknowns of the
-// 2000-bus grid, per iteration: 8.6 us in FP32, 13.7 in FP64 (two lane reads per value); two rows at a time to
-// one of 16 waves in turn, a barrier and an LDS round trip per pair of pivots, it took 14 and 19 us. With four
-// instances per workgroup (118 buses, 4 waves) each wave takes one: 6 us instead of 15 for all four.
-// Out of line: inlined, its registers and the walks' add up to spills in both.
-// ---------------------------------------------------------------------------
-template <typename FT, int G, int M>
-__device__ __noinline__ bool tail_wave(int m_, int g_, const int* src_) {
-    typedef __attribute__((address_space(3))) FT lds_ft;
-    typedef __attribute__((address_space(1))) const int glb_int;
-    const int m = __builtin_amdgcn_readfirstlane(m_), g = __builtin_amdgcn_readfirstlane(g_);
-    const int lane = threadIdx.x & 63, k0 = M - m;
-    const glb_int* const src = (const glb_int*)uniform((int*)src_) + (pfgpu::kMaxTail - M) + lane;
-    auto at = [&](int x) -> lds_ft* { return (lds_ft*)(size_t)(unsigned)(((2 * G) * (x >> 1) + 2 * g + (x & 1)) * (int)sizeof(FT)); };
-    FT R[M], Y;
-    int from[M];
-#pragma unroll
-    for (int j = 0; j < M; ++j) from[j] = src[max(j - k0, 0) * 64];
-    const int ys = src[m * 64];
-#pragma unroll
-    for (int j = 0; j < M; ++j) R[j] = *at(from[j]);
-    Y = *at(ys);
-#pragma unroll
-    for (int j = 0; j < M; ++j)
-        if (j < M - 8) R[j] = j >= k0 ? R[j] : lane == j ? (FT)1 : (FT)0;
-    bool bad = false;
-    FT D = (FT)0, r = pivot_recip(lane_read(R[0], 0));  // lane k: the reciprocal of pivot k; this pivot's
-#pragma unroll
-    for (int k = 0; k < M; ++k) {
-        bad |= bad_pivot(lane_read(R[k], k));
-        D = lane == k ? r : D;
-        const FT l = lane > k ? R[k] * r : (FT)0;
-        if (k + 1 < M) {
-            R[k + 1] -= l * lane_read(R[k + 1], k);
-            r = pivot_recip(lane_read(R[k + 1], k + 1));
-        }
-        // four lane reads, then four updates: a value just read by lane may not be used at once
-#pragma unroll
-        for (int j = k + 2; j < M; j += 4) {
-            FT u[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                if (j + i < M) u[i] = lane_read(R[j + i], k);
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                if (j + i < M) R[j + i] -= l * u[i];
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        Y -= l * lane_read(Y, k);
-    }
-    FT x = (FT)0;
-#pragma unroll
-    for (int k = M - 1; k >= 0; --k) {
-        const FT xk = lane_read(Y, k) * lane_read(D, k);
-        x = lane == k ? xk : x;
-        Y -= xk * R[k];  // (lanes from k on are done)
-    }
-    if (lane >= k0 && lane < M) *at(ys) = x;
-    return bad;
-}
-
 // v of the lane D lanes below (a sum towards the higher lanes: their last lane is the team's leader).
 // Below 16: within rows of 16 lanes, by DPP; lanes whose source lies outside the row get 0. With LAST, in steps
 // of 16 and 32 every lane gets the value of the last lane of the row (of the 32 lanes) below instead, which is
@@ -835,13 +756,7 @@ __global__ void __launch_bounds__(NT) k_nr_block(const BArgs a) {
         tmark(1);
         // ---- dense tail ---------------------------------------------------------------------------
         if (m > 0) {
-            for (int gi = wave; gi < G; gi += kWaves) {
-                if (s_done[gi]) continue;
-                const bool tbad = m <= 16   ? tail_wave<FT, G, 16>(m, gi, a.tail_src)
-                                  : m <= 32 ? tail_wave<FT, G, 32>(m, gi, a.tail_src)
-                                            : tail_wave<FT, G, 48>(m, gi, a.tail_src);
-                if (tbad) s_piv[gi] = 1;
-            }
+            tail_by_waves<TailPairs<G>, FT, G, NT>(m, a.tail_src, s_done, s_piv);
             __syncthreads();
         }
         tmark(2);

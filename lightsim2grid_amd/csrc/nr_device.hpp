@@ -6,6 +6,8 @@
 
 #include <climits>
 
+#include "blocks.hpp"
+
 namespace {
 
 constexpr int kMaxEdits = 8;  // Ybus edits per instance kept in LDS
@@ -200,6 +202,123 @@ __device__ __forceinline__ double lane_read(double v, int lane) {
 template <typename FT>
 __device__ __forceinline__ bool bad_pivot(FT v) { return !(fabs(v) > (FT)0 && fabs(v) < (FT)INFINITY); }
 
+// A pointer that is the same in every lane (one instance per workgroup), in scalar registers.
+template <typename T>
+__device__ __forceinline__ T* uniform(T* p) {
+    const unsigned long long v = (unsigned long long)p;
+    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)v), hi = __builtin_amdgcn_readfirstlane((unsigned)(v >> 32));
+    return (T*)((unsigned long long)hi << 32 | lo);
+}
+
+// Where a tail's numbers lie: the FT at (row `lane`, column c) of instance g, in units of FT; column m is the
+// right-hand side. On the block plan by a table, by columns of 64 lanes (2 pair + component); else as a tile,
+// row-major, stride m + 1, from slot 0 on. Lanes past the rows name a number that is there.
+template <int G>
+struct TailPairs {
+    typedef __attribute__((address_space(1))) const int* src_t;
+    int m, g;
+    src_t src;
+    __device__ __forceinline__ int operator()(int, int c) const {
+        const int x = src[c * 64];
+        return (2 * G) * (x >> 1) + 2 * g + (x & 1);
+    }
+};
+template <int G>
+struct TailTile {
+    typedef __attribute__((address_space(1))) const int* src_t;
+    int m, g;
+    src_t src;
+    __device__ __forceinline__ int operator()(int lane, int c) const { return (min(lane, m - 1) * (m + 1) + c) * G + g; }
+};
+
+// ---------------------------------------------------------------------------
+// Dense tail of one instance (m <= kMaxTail unknowns) on one wave, in registers: lane = row, R[j] = the j-th
+// column that is left, Y = the right-hand side. A step eliminates the pivot's column from every other row,
+// those above it too (Gauss-Jordan: their lanes are there anyway, and no backward sweep follows), and moves the
+// columns one register down, so that it is a loop: unrolled over the pivots its FP64 form is 50 KB of code,
+// which with the walks does not stay in the instruction cache. The pivot row reaches the other lanes by lane
+// reads of each column, the next pivot's first, whose reciprocal is then formed beside the other columns'
+// updates; no LDS access and no barrier lies between the pivots. A loop each for the last 8, 16, .. 48 columns.
+// Where: where the numbers lie in LDS, from address 0 on; the right-hand side's places receive the solution.
+// Returns whether a pivot was zero or non-finite.
+// Bound by the instruction issue of one wave: about m^2 / 2 lane reads and as many updates. 43 unknowns of the
+// 2000-bus grid, per iteration: 9.8 us in FP32, 15.6 in FP64 (two lane reads per value); two rows at a time to
+// one of 16 waves in turn, a barrier and an LDS round trip per pair of pivots, it took 14 and 19 us. Unrolled it
+// takes 1 us less, but the kernel is slower where factor levels are short (613-bus N-2: 437 against 410 us).
+// With four instances per workgroup (118 buses, 4 waves) each wave takes one: 8 us instead of 15 for all four.
+// Out of line: inlined, its registers and the walks' add up to spills in both.
+// ---------------------------------------------------------------------------
+template <int W, typename FT>
+__device__ __forceinline__ void tail_steps(FT (&R)[pfgpu::kMaxTail], FT& Y, FT& D, FT& r, int& k, int m, int lane, bool& bad) {
+    if constexpr (W > 0) {
+        while (k < m && m - k > W - 8) {  // R[0 .. W - 1] hold what is left
+            bad |= bad_pivot(lane_read(R[0], k));
+            D = lane == k ? r : D;
+            const FT l = lane == k ? (FT)0 : R[0] * r;
+            const FT u0 = lane_read(R[1], k), uy = lane_read(Y, k);
+            R[0] = R[1] - l * u0;
+            r = pivot_recip(lane_read(R[0], k + 1));
+            Y -= l * uy;
+            // four lane reads, then four updates: a value just read by lane may not be used at once
+#pragma unroll
+            for (int j = 1; j + 1 < W; j += 4) {
+                FT u[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (j + i + 1 < W) u[i] = lane_read(R[j + i + 1], k);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (j + i + 1 < W) R[j + i] = R[j + i + 1] - l * u[i];
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            ++k;
+        }
+        tail_steps<W - 8>(R, Y, D, r, k, m, lane, bad);
+    }
+}
+
+template <class Where, typename FT>
+__device__ __noinline__ bool tail_wave(int m_, int g_, const int* src_) {
+    typedef __attribute__((address_space(3))) FT lds_ft;
+    constexpr int M = pfgpu::kMaxTail;
+    const int m = __builtin_amdgcn_readfirstlane(m_), g = __builtin_amdgcn_readfirstlane(g_);
+    const int lane = threadIdx.x & 63;
+    const Where where{m, g, (typename Where::src_t)(uniform((int*)src_) + lane)};
+    auto at = [&](int i) -> lds_ft* { return (lds_ft*)(size_t)(unsigned)(i * (int)sizeof(FT)); };
+    FT R[M], Y;
+    int from[M];
+    const int ys = where(lane, m);
+#pragma unroll
+    for (int c = 0; c < M; c += 8)
+        if (c < m)
+#pragma unroll
+            for (int j = c; j < c + 8; ++j) from[j] = where(lane, min(j, m));
+    Y = *at(ys);
+#pragma unroll
+    for (int c = 0; c < M; c += 8)
+        if (c < m) {
+#pragma unroll
+            for (int j = c; j < c + 8; ++j) R[j] = *at(from[j]);
+#pragma unroll
+            for (int j = c; j < c + 8; ++j) R[j] = lane < m ? R[j] : (FT)0;
+        }
+    bool bad = false;
+    FT D = (FT)0, r = pivot_recip(lane_read(R[0], 0));  // lane k: the reciprocal of pivot k; this pivot's
+    int k = 0;
+    tail_steps<M>(R, Y, D, r, k, m, lane, bad);
+    if (lane < m) *at(ys) = Y * D;
+    return bad;
+}
+
+// The tails of a workgroup's G instances (m <= kMaxTail), an instance to a wave.
+template <class Where, typename FT, int G, int NT, typename LI>
+__device__ __forceinline__ void tail_by_waves(int m, const int* src, LI done, LI piv) {
+    for (int g = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); g < G; g += NT / 64) {
+        if (done[g]) continue;
+        if (tail_wave<Where, FT>(m, g, src)) piv[g] = 1;
+    }
+}
 
 // ---- dense tail: the m x m tile of every instance ---------------------------------
 // Tile at slots [0, m*(m+1)): row-major with row stride m + 1, the right-hand side

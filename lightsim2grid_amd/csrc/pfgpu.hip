@@ -385,29 +385,10 @@ __global__ void __launch_bounds__(NT) k_nr(const KArgs a) {
     // load before them, coalesced across lanes, and summed in row order.
     auto mismatch = [&]() -> double {
         double fm = 0.0;
-        if (run && !s_done[g] && a.dc) {
-            // DC: F = Re(Y) theta - Re(S) over the non-slack columns; fm = max |theta| of the rows
-            EditPos dp;
-            edit_pos(dp);
+        if (run && !s_done[g] && a.dc) {  // DC: the largest |theta| of the rows
             const double vas = Va[a.slack0];
-            for (int r = s; r < n; r += nslot) {
-                const int len = a.yr_ptr[r + 1] - a.yr_ptr[r];
-                const int fp = a.fslot_p[r];
-                double acc = 0.0;
-                for (int k0 = 0; k0 == 0 || k0 < len; k0 += kEll) {
-#pragma unroll
-                    for (int k = 0; k < kEll; ++k) {
-                        const int2 pc = a.yr_ell[(size_t)(k0 + k) * n + r];
-                        if (pc.x < 0 || a.bus_dx[pc.y].x < 0) continue;
-                        const c64 yv = Yell ? edits(ld_c(Yell, (k0 + k) * n + r), pc.x, dp) : Yat(pc.x, dp);
-                        acc += yv.re * (Va[pc.y] - vas);
-                    }
-                }
-                if (fp >= 0) {
-                    XS(fp, (FT)(acc - S[2 * r]));
-                    fm = fmax(fm, inf_if_nonfinite(fabs(Va[r] - vas)));
-                }
-            }
+            for (int r = s; r < n; r += nslot)
+                if (a.fslot_p[r] >= 0) fm = fmax(fm, inf_if_nonfinite(fabs(Va[r] - vas)));
         } else if (run && !s_done[g]) {
             const double sa = s_slack[g];
             EditPos dp;
@@ -452,7 +433,46 @@ __global__ void __launch_bounds__(NT) k_nr(const KArgs a) {
         return inst_reduce<G, NT, true>(fm, s_part);
     };
 
-    double fmx = mismatch();
+    // DC: F = Re(Y) theta - Re(S) over the non-slack columns. A row's entries are read kEll at a time in two
+    // round trips, {table, Ybus value} and {theta, unknown} of the column; entry by entry behind tests they
+    // took three each (2000-bus DC N-1: 443 -> 220 us of a workgroup's 1000, instance setup included, together
+    // with the |theta| pass above, which took the whole sum once more).
+    auto dc_rhs = [&]() {
+        if (!run || s_done[g]) return;
+        EditPos dp;
+        edit_pos(dp);
+        const double vas = Va[a.slack0];
+        for (int r = s; r < n; r += nslot) {
+            const int len = a.yr_ptr[r + 1] - a.yr_ptr[r];
+            const int fp = a.fslot_p[r];
+            const double sr = S[2 * r];
+            double acc = 0.0;
+            for (int k0 = 0; k0 == 0 || k0 < len; k0 += kEll) {
+                int2 pc[kEll];
+                double yv[kEll], th[kEll];
+                int dx[kEll];
+#pragma unroll
+                for (int k = 0; k < kEll; ++k) {
+                    pc[k] = a.yr_ell[(size_t)(k0 + k) * n + r];
+                    if (Yell) yv[k] = Yell[2 * ((size_t)(k0 + k) * n + r)];
+                }
+#pragma unroll
+                for (int k = 0; k < kEll; ++k) {
+                    if (!Yell) yv[k] = Y[2 * (size_t)max(pc[k].x, 0)];
+                    th[k] = Va[pc[k].y] - vas;
+                    dx[k] = a.bus_dx[pc[k].y].x;
+                }
+#pragma unroll
+                for (int k = 0; k < kEll; ++k)
+                    if (pc[k].x >= 0 && dx[k] >= 0) acc += edits(c64{yv[k], 0.0}, pc[k].x, dp).re * th[k];
+            }
+            if (fp >= 0) XS(fp, (FT)(acc - sr));
+        }
+    };
+
+    double fmx = 0.0;
+    if (a.dc) dc_rhs();
+    else fmx = mismatch();
     if (s == 0 && run && !s_done[g] && !a.dc) {  // DC: always one linear solve
         s_flast[g] = fmx;
         if (fmx < a.tol) s_done[g] = 1;  // converged at iteration 0
@@ -774,9 +794,13 @@ __global__ void __launch_bounds__(NT) k_nr(const KArgs a) {
         tmark(1);
         // ---- dense tail: the m x m tile of every instance ---------------------------------
         if (a.m > 0) {
-            bool bad_t = false;
-            dense_tail_lds<FT, G, NT>(Xl, a.m, g, s, act, bad_t);
-            if (bad_t && s == 0) s_piv[g] = 1;
+            if (a.m <= pfgpu::kMaxTail) {
+                tail_by_waves<TailTile<G>, FT, G, NT>(a.m, nullptr, s_done, s_piv);
+            } else {
+                bool bad_t = false;
+                dense_tail_lds<FT, G, NT>(Xl, a.m, g, s, act, bad_t);
+                if (bad_t && s == 0) s_piv[g] = 1;
+            }
             __syncthreads();
         }
         tmark(2);
@@ -1561,8 +1585,8 @@ LaunchChoice choose_launch(const pfgpu_ctx* ctx, const pfgpu::DevicePlan& P, int
     // lean: every value slot in LDS, and the instances' V beside them
     c.lean = c.nspill == 0 && c.v_off + (size_t)P.n * c.G * 16 <= (size_t)ctx->lds_max;
     // lean items carry LDS addresses: the value slots must start at LDS address 0
-    if (c.lean && static_lds(fsize, c.G, c.NT) != 0)
-        throw ApiError(PFGPU_E_INTERNAL, "the NR kernel has static LDS: lean item offsets would not be LDS addresses");
+    if (static_lds(fsize, c.G, c.NT) != 0)
+        throw ApiError(PFGPU_E_INTERNAL, "the NR kernel has static LDS: lean items and the tail would not find their values");
     c.nblocks = (ninst + c.G - 1) / c.G;
     c.lds = c.lean ? c.v_off + (size_t)P.n * c.G * 16 : c.v_off;
     return c;
@@ -2647,11 +2671,10 @@ std::unique_ptr<pfgpu_grid::Block> upload_blocks(const pfgpu_grid* g, const std:
         d.upload(v);
     };
     b->bus_y.upload(B.bus_y);
-    // by columns, a lane per row: rows and columns end at kMaxTail, lanes beside them read a zero (a wave on M
-    // of the columns starts kMaxTail - M lanes into the first, and so ends within one more)
-    std::vector<int> tail(B.m > 0 ? (size_t)(B.m + 2) * 64 : 0, 2 * B.zpair);
+    // by columns, a lane per row
+    std::vector<int> tail(B.m > 0 ? (size_t)(B.m + 1) * 64 : 0, 2 * B.zpair);
     for (int r = 0; r < B.m; ++r)
-        for (int c = 0; c <= B.m; ++c) tail[(size_t)c * 64 + (pfgpu::kMaxTail - B.m + r)] = B.tail_src[(size_t)r * (B.m + 1) + c];
+        for (int c = 0; c <= B.m; ++c) tail[(size_t)c * 64 + r] = B.tail_src[(size_t)r * (B.m + 1) + c];
     up(b->tail_src, tail);
     b->y_row.upload(g->Y.i);
     const int nrow = (int)B.row_len.size(), nent = (int)B.jd_pos.size();
