@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <functional>
 #include <mutex>
 #include <stdexcept>
 #include <string>
@@ -72,6 +73,13 @@ struct pfgpu_ctx {
     // two-pass single chains: the first pass's rows, the second pass's starts, flags (grow-only)
     void* chain = nullptr;
     size_t chain_bytes = 0;
+    // pinned host memory: the head of aux as the last launch left it (fallback count, phase clocks), and the
+    // staging of the small host-buffer solves (grow-only, at most kPinMax)
+    char* head = nullptr;
+    void* pin = nullptr;
+    size_t pin_bytes = 0;
+    // work to put on the stream after the next launch, before the wait for it (set and taken under mu)
+    std::function<void()> before_sync;
     long long last_rows = 0;            // rows of the last solve call
     const int* last_flags = nullptr;    // and their flags (device)
     hipEvent_t ev0 = nullptr, ev1 = nullptr;

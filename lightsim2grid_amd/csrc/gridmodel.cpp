@@ -573,22 +573,47 @@ void BaseBatchSolverSynch::compute_flows_from_Vs(bool amps) {
     IntVect cptr, cbr;
     clean_lists(cptr, cbr);
     const bool clean = !cbr.empty();
-    int* df = d_tmp_[0].upload(f);
-    int* dt = d_tmp_[1].upload(t);
-    double* dyff = reinterpret_cast<double*>(d_tmp_[2].upload(yff));
-    double* dyft = reinterpret_cast<double*>(d_tmp_[3].upload(yft));
-    double* dvn = d_tmp_[4].upload(vn);
-    int* dcp = clean ? d_tmp_[5].upload(cptr) : nullptr;
-    int* dcb = clean ? d_tmp_[6].upload(cbr) : nullptr;
-    RealVect& out = amps ? amps_ : pflows_;
-    out.assign((size_t)nrows_ * nl, 0.0);
+    Pack pk;
+    const size_t o_f = pk.add(f), o_t = pk.add(t), o_ff = pk.add(yff), o_ft = pk.add(yft), o_vn = pk.add(vn);
+    const size_t o_cp = pk.add(cptr), o_cb = pk.add(cbr);
+    char* const b = pk.upload(d_tmp_[0]);
+    int *df = reinterpret_cast<int*>(b + o_f), *dt = reinterpret_cast<int*>(b + o_t);
+    double *dyff = reinterpret_cast<double*>(b + o_ff), *dyft = reinterpret_cast<double*>(b + o_ft);
+    double* dvn = reinterpret_cast<double*>(b + o_vn);
+    int *dcp = clean ? reinterpret_cast<int*>(b + o_cp) : nullptr, *dcb = clean ? reinterpret_cast<int*>(b + o_cb) : nullptr;
+    RealRows& out = amps ? amps_ : pflows_;
+    out.resize((size_t)nrows_ * nl);  // (every number is written by the kernel)
     double* dout = static_cast<double*>(d_tmp_[7].get(std::max<size_t>(out.size(), 1) * 8));
     auto flows = dc_rows_ ? pfgpu_batch_flows_dc_device : pfgpu_batch_flows_device;
-    check_rc(flows(engine_ctx(), nrows_, ns_, d_V_.as<double>(), d_row_src_.as<int>(), nl, df, dt, dyff, dyft, dvn,
-                   grid_model_.get_sn_mva(), dcp, dcb, amps ? dout : nullptr, amps ? nullptr : dout),
-             dc_rows_ ? "pfgpu_batch_flows_dc_device" : "pfgpu_batch_flows_device");
-    if (!out.empty()) check_rc(pfgpu_memcpy_d2h(engine_ctx(), out.data(), dout, out.size() * 8), "d2h");
+    try {
+        check_rc(flows(engine_ctx(), nrows_, ns_, d_V_.as<double>(), d_row_src_.as<int>(), nl, df, dt, dyff, dyft, dvn,
+                       grid_model_.get_sn_mva(), dcp, dcb, amps ? dout : nullptr, amps ? nullptr : dout),
+                 dc_rows_ ? "pfgpu_batch_flows_dc_device" : "pfgpu_batch_flows_device");
+        if (!out.empty()) check_rc(pfgpu_memcpy_d2h(engine_ctx(), out.data(), dout, out.size() * 8), "d2h");
+    } catch (...) {
+        out.clear();
+        throw;
+    }
     if (amps) timer_amps_ = since(t0);
+}
+
+void BaseBatchSolverSynch::take_voltages(const double* d_V, int nsolved, const IntVect& to, const IntVect& bus, int nb) {
+    const int ns = (int)bus.size(), rows = nrows_;
+    voltages_.resize((size_t)rows * nb);
+    bool straight = ns == nb && nsolved == rows;  // row by row and bus by bus as the device has them
+    for (int b = 0; b < ns && straight; ++b) straight = bus[b] == b;
+    if (straight) {
+        if (rows > 0) check_rc(pfgpu_memcpy_d2h(engine_ctx(), voltages_.data(), d_V, voltages_.size() * 16), "d2h");
+        for (int r = 0; r < rows; ++r)
+            if (to[r] != r) std::fill_n(voltages_.begin() + (size_t)r * nb, nb, cplx(0, 0));
+        return;
+    }
+    std::fill(voltages_.begin(), voltages_.end(), cplx(0, 0));
+    CplxRows got((size_t)nsolved * ns);
+    if (nsolved > 0) check_rc(pfgpu_memcpy_d2h(engine_ctx(), got.data(), d_V, got.size() * 16), "d2h");
+    for (int r = 0; r < nsolved; ++r)
+        if (to[r] >= 0)
+            for (int b = 0; b < ns; ++b) voltages_[(size_t)to[r] * nb + bus[b]] = got[(size_t)r * ns + b];
 }
 
 void ContingencyAnalysis::add_all_n1() {
@@ -741,9 +766,9 @@ void ContingencyAnalysis::compute(const CplxVect& Vinit, int max_iter, double to
     nrows_ = ncont;
     ns_ = 0;
     id_me_to_solver_ = in.id_me_to_solver;
-    voltages_.assign((size_t)ncont * nb, cplx(0, 0));
     amps_.clear();
     pflows_.clear();
+    ZerosUnlessTaken volts{*this, (size_t)nrows_ * nb, false};
     GpuNRSolver& s = solver_.current();
     dc_rows_ = dc;
     s.reset();
@@ -764,22 +789,21 @@ void ContingencyAnalysis::compute(const CplxVect& Vinit, int max_iter, double to
     const int n = in.Ybus.ncol;
     pfgpu_ctx* ctx = engine_ctx();
     IntVect conn(ncont, dc ? 1 : 0);
-    DevMem m[9];
-    double* dYx = reinterpret_cast<double*>(d_Y_.upload(in.Ybus.x));
-    int* dpos_br = m[2].upload(pos);
-    double* dy = reinterpret_cast<double*>(m[3].upload(y));
+    Pack pk;
+    const size_t o_yx = pk.add(in.Ybus.x), o_pos = pk.add(pos), o_y = pk.add(y), o_ptr = pk.add(all.ptr), o_br = pk.add(all.br);
+    const size_t o_dp = pk.add(all.dptr), o_yp = pk.add(in.Ybus.p), o_yi = pk.add(in.Ybus.i);
+    char* const b0 = pk.upload(d_tmp_[3]);
+    double *dYx = reinterpret_cast<double*>(b0 + o_yx), *dy = reinterpret_cast<double*>(b0 + o_y);
+    int* dpos_br = reinterpret_cast<int*>(b0 + o_pos);
     if (ncont > 0 && !dc) {
-        int* dcp = m[0].upload(all.ptr);
-        int* dcb = m[1].upload(all.br);
-        int* ddp = m[4].upload(all.dptr);
-        int* ddq = static_cast<int*>(m[5].get(std::max(all.dptr.back(), 1) * sizeof(int)));
-        double* ddv = static_cast<double*>(m[6].get(std::max(all.dptr.back(), 1) * 16));
+        int *dcp = reinterpret_cast<int*>(b0 + o_ptr), *dcb = reinterpret_cast<int*>(b0 + o_br);
+        int* ddp = reinterpret_cast<int*>(b0 + o_dp);
+        int* ddq = static_cast<int*>(d_tmp_[1].get(std::max(all.dptr.back(), 1) * sizeof(int)));
+        double* ddv = static_cast<double*>(d_tmp_[2].get(std::max(all.dptr.back(), 1) * 16));
         check_rc(pfgpu_contingency_edits_device(ctx, ncont, dcp, dcb, dpos_br, dy, ddp, ddq, ddv),
                  "pfgpu_contingency_edits_device");
-        int* dYp = m[7].upload(in.Ybus.p);
-        int* dYi = m[8].upload(in.Ybus.i);
-        DevMem mc;
-        int* dconn = static_cast<int*>(mc.get(ncont * sizeof(int)));
+        int *dYp = reinterpret_cast<int*>(b0 + o_yp), *dYi = reinterpret_cast<int*>(b0 + o_yi);
+        int* dconn = static_cast<int*>(d_tmp_[5].get(ncont * sizeof(int)));
         check_rc(pfgpu_connectivity_device(ctx, ncont, n, dYp, dYi, dYx, ddp, ddq, ddv, dconn),
                  "pfgpu_connectivity_device");
         check_rc(pfgpu_memcpy_d2h(ctx, conn.data(), dconn, ncont * sizeof(int)), "d2h");
@@ -798,41 +822,40 @@ void ContingencyAnalysis::compute(const CplxVect& Vinit, int max_iter, double to
         }
     }
     const int m_solve = (int)which.size();
-    int* sdp = d_tmp_[0].upload(sel.dptr);
+    Pack ps;
+    const size_t o_sdp = ps.add(sel.dptr), o_sp = ps.add(sel.ptr), o_sb = ps.add(sel.br), o_s = ps.add(in.Sbus);
+    const size_t o_v0 = ps.add(Vstart);
+    char* const b1 = ps.upload(d_tmp_[4]);
+    int* sdp = reinterpret_cast<int*>(b1 + o_sdp);
     int* sdq = static_cast<int*>(d_tmp_[1].get(std::max(sel.dptr.back(), 1) * sizeof(int)));
     double* sdv = static_cast<double*>(d_tmp_[2].get(std::max(sel.dptr.back(), 1) * 16));
     if (m_solve > 0) {
-        int* scp = m[0].upload(sel.ptr);
-        int* scb = m[1].upload(sel.br);
+        int *scp = reinterpret_cast<int*>(b1 + o_sp), *scb = reinterpret_cast<int*>(b1 + o_sb);
         check_rc(pfgpu_contingency_edits_device(ctx, m_solve, scp, scb, dpos_br, dy, sdp, sdq, sdv),
                  "pfgpu_contingency_edits_device");
     }
     timer_modif_ybus_ = since(t_y);
     // batched solve, tol / sn_mva (ContingencyAnalysis.cpp:223)
     auto t_s = clk::now();
-    double* dS = reinterpret_cast<double*>(d_S_.upload(in.Sbus));
-    double* dV0 = reinterpret_cast<double*>(d_V0_.upload(Vstart));
+    double *dS = reinterpret_cast<double*>(b1 + o_s), *dV0 = reinterpret_cast<double*>(b1 + o_v0);
     double* dV = static_cast<double*>(d_V_.get((size_t)std::max(m_solve, 1) * ns * 16));
     int* dIt = static_cast<int*>(d_iters_.get((size_t)std::max(m_solve, 1) * sizeof(int)));
     int* dSt = static_cast<int*>(d_status_.get((size_t)std::max(m_solve, 1) * sizeof(int)));
     pfgpu_stats st{};
     s.solve_batch_device(in.Ybus, in.slack_ids, in.slack_weights, in.pv, in.pq, m_solve, dYx, sdp, sdq, sdv, dS, false,
                          dV0, false, dV, max_iter, tol / sn, dIt, dSt, &st);
-    CplxVect Vout((size_t)m_solve * ns);
     IntVect status(m_solve);
-    if (m_solve > 0) {
-        check_rc(pfgpu_memcpy_d2h(ctx, Vout.data(), dV, Vout.size() * 16), "d2h");
-        check_rc(pfgpu_memcpy_d2h(ctx, status.data(), dSt, status.size() * sizeof(int)), "d2h");
-    }
-    timer_solver_ += since(t_s);
+    if (m_solve > 0) check_rc(pfgpu_memcpy_d2h(ctx, status.data(), dSt, status.size() * sizeof(int)), "d2h");
     nb_solved_ = m_solve;
-    IntVect row_src(ncont, -1);
+    IntVect row_src(ncont, -1), to(m_solve, -1);
     for (int w = 0; w < m_solve; ++w) {
         if (status[w] != 0) continue;
-        const int row = which[w];
-        row_src[row] = w;
-        for (int b = 0; b < ns; ++b) voltages_[(size_t)row * nb + in.id_solver_to_me[b]] = Vout[(size_t)w * ns + b];
+        to[w] = which[w];
+        row_src[which[w]] = w;
     }
+    take_voltages(dV, m_solve, to, in.id_solver_to_me, nb);
+    volts.taken = true;
+    timer_solver_ += since(t_s);
     keep_device_rows(ns, row_src);
     timer_total_ = since(t_all);
 }
@@ -852,16 +875,15 @@ void TimeSeries::clear() {
 // side, each chain head starting from the initial V. With the DC solver every step is solved from
 // the initial V side by side: a DC solve sets the angles from B theta = P alone and keeps the
 // magnitudes of its initial V, so a step's result does not depend on the step before it.
-int TimeSeries::compute_Vs(int T, const RealVect& gen_p, const RealVect& sgen_p, const RealVect& load_p,
-                           const RealVect& load_q, const CplxVect& Vinit, int max_iter, double tol) {
+int TimeSeries::compute_Vs(int T, const RealView& gen_p, const RealView& sgen_p, const RealView& load_p,
+                           const RealView& load_q, const CplxVect& Vinit, int max_iter, double tol) {
     auto t_all = clk::now();
     auto t_pre = clk::now();
     status_ = 0;
     nb_solved_ = 0;
     timer_solver_ = 0;
     const int ng = grid_model_.nb_gen(), nsg = grid_model_.nb_sgen(), nl = grid_model_.nb_load();
-    if ((int)gen_p.size() != T * ng || (int)sgen_p.size() != T * nsg || (int)load_p.size() != T * nl ||
-        (int)load_q.size() != T * nl)
+    if ((int)gen_p.n != T * ng || (int)sgen_p.n != T * nsg || (int)load_p.n != T * nl || (int)load_q.n != T * nl)
         throw std::runtime_error("TimeSeries::compute_Vs: injection matrices must be [T x nb_element]");
     const double sn = grid_model_.get_sn_mva();
     const bool dc = solver_.current().is_dc();
@@ -886,18 +908,26 @@ int TimeSeries::compute_Vs(int T, const RealVect& gen_p, const RealVect& sgen_p,
     lists(nsg, [&](int e) { return grid_model_.sgen_bus(e); }, sp, se);
     lists(nl, [&](int e) { return grid_model_.load_bus(e); }, lp, le);
     pfgpu_ctx* ctx = engine_ctx();
-    DevMem m[10];
     double* dS = static_cast<double*>(d_S_.get((size_t)std::max(T, 1) * ns * 16));
-    check_rc(pfgpu_sbus_rows_device(ctx, T, ns, m[0].upload(gp), m[1].upload(ge), ng, m[2].upload(gen_p),
-                                    m[3].upload(sp), m[4].upload(se), nsg, m[5].upload(sgen_p), m[6].upload(lp),
-                                    m[7].upload(le), nl, m[8].upload(load_p), m[9].upload(load_q), sn, dS),
+    Pack pk;
+    const size_t o[6] = {pk.add(gp), pk.add(ge), pk.add(sp), pk.add(se), pk.add(lp), pk.add(le)};
+    char* const b0 = pk.upload(d_in_[0]);
+    auto ids = [&](int k) { return reinterpret_cast<const int*>(b0 + o[k]); };
+    auto rows = [&](DevMem& m, const RealView& v) {
+        double* d = static_cast<double*>(m.get(std::max<size_t>(v.n, 1) * sizeof(double)));
+        if (v.n) check_rc(pfgpu_memcpy_h2d(ctx, d, v.p, v.n * sizeof(double)), "h2d");
+        return d;
+    };
+    check_rc(pfgpu_sbus_rows_device(ctx, T, ns, ids(0), ids(1), ng, rows(d_in_[1], gen_p), ids(2), ids(3), nsg,
+                                    rows(d_in_[2], sgen_p), ids(4), ids(5), nl, rows(d_in_[3], load_p),
+                                    rows(d_in_[4], load_q), sn, dS),
              "pfgpu_sbus_rows_device");
-    sbuses_.assign((size_t)T * ns, cplx(0, 0));
+    sbuses_.resize((size_t)T * ns);
     if (T > 0) check_rc(pfgpu_memcpy_d2h(ctx, sbuses_.data(), dS, sbuses_.size() * 16), "d2h");
     nrows_ = T;
-    voltages_.assign((size_t)T * nb, cplx(0, 0));
     amps_.clear();
     pflows_.clear();
+    ZerosUnlessTaken volts{*this, (size_t)nrows_ * nb, false};
     GpuNRSolver& s = solver_.current();
     dc_rows_ = dc;
     s.reset();
@@ -909,30 +939,27 @@ int TimeSeries::compute_Vs(int T, const RealVect& gen_p, const RealVect& sgen_p,
     const CplxVect Vstart = init_from_n_ ? s.get_V() : in.V;
     const int L = dc ? 1 : std::max(1, std::min(chain_len_ > 0 ? chain_len_ : T, std::max(T, 1)));
     auto t_s = clk::now();
-    double* dYx = reinterpret_cast<double*>(d_Y_.upload(in.Ybus.x));
-    double* dV0 = reinterpret_cast<double*>(d_V0_.upload(Vstart));
+    Pack ps;
+    const size_t o_yx = ps.add(in.Ybus.x), o_v0 = ps.add(Vstart);
+    char* const b1 = ps.upload(d_tmp_[4]);
+    double *dYx = reinterpret_cast<double*>(b1 + o_yx), *dV0 = reinterpret_cast<double*>(b1 + o_v0);
     double* dV = static_cast<double*>(d_V_.get((size_t)std::max(T, 1) * ns * 16));
     int* dIt = static_cast<int*>(d_iters_.get((size_t)std::max(T, 1) * sizeof(int)));
     int* dSt = static_cast<int*>(d_status_.get((size_t)std::max(T, 1) * sizeof(int)));
     pfgpu_stats st{};
     s.solve_chains_device(in.Ybus, in.slack_ids, in.slack_weights, in.pv, in.pq, T, L, dYx, dS, dV0, dV, max_iter,
                           tol / sn, dIt, dSt, &st);
-    CplxVect Vout((size_t)T * ns);
     IntVect stt(T);
-    if (T > 0) {
-        check_rc(pfgpu_memcpy_d2h(ctx, Vout.data(), dV, Vout.size() * 16), "d2h");
-        check_rc(pfgpu_memcpy_d2h(ctx, stt.data(), dSt, stt.size() * sizeof(int)), "d2h");
-    }
-    timer_solver_ += since(t_s);
+    if (T > 0) check_rc(pfgpu_memcpy_d2h(ctx, stt.data(), dSt, stt.size() * sizeof(int)), "d2h");
     // the reference stops at the first divergence (TimeSeries.cpp:94-99)
     int first_fail = T;
     for (int t = 0; t < T; ++t)
         if (stt[t] != 0) { first_fail = t; break; }
     IntVect row_src(T, -1);
-    for (int t = 0; t < first_fail; ++t) {
-        row_src[t] = t;
-        for (int b = 0; b < ns; ++b) voltages_[(size_t)t * nb + in.id_solver_to_me[b]] = Vout[(size_t)t * ns + b];
-    }
+    for (int t = 0; t < first_fail; ++t) row_src[t] = t;
+    take_voltages(dV, T, row_src, in.id_solver_to_me, nb);
+    volts.taken = true;
+    timer_solver_ += since(t_s);
     keep_device_rows(ns, row_src);
     nb_solved_ = std::min(T, first_fail + 1);
     status_ = first_fail == T ? 1 : 0;

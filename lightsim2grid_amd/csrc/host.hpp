@@ -15,6 +15,7 @@
 #include <algorithm>
 #include <complex>
 #include <cstdint>
+#include <cstring>
 #include <memory>
 #include <set>
 #include <stdexcept>
@@ -97,6 +98,42 @@ private:
     void* p_ = nullptr;
     size_t n_ = 0;
 };
+
+// Arrays for the device gathered on the host, for one copy into one buffer.
+class Pack {
+public:
+    // offset of v's copy in the buffer
+    template <class T>
+    size_t add(const std::vector<T>& v) {
+        const size_t at = (h_.size() + 15) & ~(size_t)15;
+        h_.resize(at + std::max<size_t>(v.size(), 1) * sizeof(T));
+        if (!v.empty()) std::memcpy(h_.data() + at, v.data(), v.size() * sizeof(T));
+        return at;
+    }
+    char* upload(DevMem& m) const { return m.upload(h_); }
+
+private:
+    std::vector<char> h_;
+};
+
+// Numbers of the caller's, read in place.
+struct RealView {
+    const double* p;
+    size_t n;
+};
+
+// Leaves new elements unwritten: for results that a copy from the device fills.
+template <class T>
+struct Unwritten : std::allocator<T> {
+    template <class U>
+    struct rebind { using other = Unwritten<U>; };
+    template <class U>
+    void construct(U*) noexcept {}
+    template <class U, class A, class... B>
+    void construct(U* p, A&& a, B&&... b) { ::new ((void*)p) U(std::forward<A>(a), std::forward<B>(b)...); }
+};
+using CplxRows = std::vector<cplx, Unwritten<cplx>>;
+using RealRows = std::vector<double, Unwritten<double>>;
 
 // ---------------------------------------------------------------------------
 // One GPU NR solver (the reference's BaseNRAlgo / BaseNRSingleSlackAlgo
@@ -314,9 +351,9 @@ public:
     double amps_computation_time() const { return timer_amps_; }
     int nb_solved() const { return nb_solved_; }
     // results, row-major [nsteps x n]
-    const CplxVect& get_voltages() const { return voltages_; }
-    const RealVect& get_flows() const { return amps_; }
-    const RealVect& get_power_flows() const { return pflows_; }
+    const CplxRows& get_voltages() const { return voltages_; }
+    const RealRows& get_flows() const { return amps_; }
+    const RealRows& get_power_flows() const { return pflows_; }
     int nb_rows() const { return nrows_; }
     int nb_bus_total() const { return grid_model_.total_bus(); }
     int nb_branch() const { return grid_model_.nb_powerline(); }
@@ -336,12 +373,30 @@ protected:
     double timer_total_ = 0, timer_solver_ = 0, timer_pre_proc_ = 0, timer_amps_ = 0;
     int nb_solved_ = 0;
     int nrows_ = 0;
-    CplxVect voltages_;
-    RealVect amps_, pflows_;
+    CplxRows voltages_;
+    RealRows amps_, pflows_;
     IntVect id_me_to_solver_;  // of the last compute
     int ns_ = 0;               // solver buses of the last compute
     bool dc_rows_ = false;     // the last compute used the DC solver (ac_solver_used() false)
-    DevMem d_V_, d_row_src_, d_iters_, d_status_, d_S_, d_Y_, d_V0_, d_tmp_[8];
+    DevMem d_V_, d_row_src_, d_iters_, d_status_, d_S_, d_tmp_[8];
+    // rows of the device voltages (bus order of the solver) into voltages_ (row `to[r]` of the grid's buses, -1:
+    // none); the other rows and buses are zero
+    void take_voltages(const double* d_V, int nsolved, const IntVect& to, const IntVect& bus, int nb);
+    // While a compute has not brought its voltages: if it ends without them, they are zeros
+    struct ZerosUnlessTaken {
+        BaseBatchSolverSynch& b;
+        size_t size;
+        bool taken;
+        ~ZerosUnlessTaken() {
+            if (taken) return;
+            try {
+                b.voltages_.assign(size, cplx(0, 0));
+            } catch (...) {  // no memory: no rows
+                b.voltages_.clear();
+                b.nrows_ = 0;
+            }
+        }
+    };
 };
 
 class ContingencyAnalysis : public BaseBatchSolverSynch {
@@ -377,12 +432,12 @@ class TimeSeries : public BaseBatchSolverSynch {
 public:
     using BaseBatchSolverSynch::BaseBatchSolverSynch;
     // gen_p [T x nb_gen], sgen_p [T x nb_sgen], load_p/load_q [T x nb_load], row-major
-    int compute_Vs(int T, const RealVect& gen_p, const RealVect& sgen_p, const RealVect& load_p, const RealVect& load_q,
+    int compute_Vs(int T, const RealView& gen_p, const RealView& sgen_p, const RealView& load_p, const RealView& load_q,
                    const CplxVect& Vinit, int max_iter, double tol);
     void compute_flows() { compute_flows_from_Vs(true); }
     void compute_power_flows() { compute_flows_from_Vs(false); }
     int get_status() const { return status_; }
-    const CplxVect& get_sbuses() const { return sbuses_; }
+    const CplxRows& get_sbuses() const { return sbuses_; }
     int nb_bus_solver() const { return nbus_solver_; }
     void clear();
     // Steps run as warm-started chains of `chain_length` steps side by side; 0 (the default) or
@@ -392,7 +447,8 @@ public:
 
 private:
     int status_ = 1;
-    CplxVect sbuses_;
+    CplxRows sbuses_;
+    DevMem d_in_[5];
     int nbus_solver_ = 0;
     int chain_len_ = 0;
 };

@@ -39,8 +39,8 @@ py::array_t<int> to_np(const IntVect& v) {
     std::copy(v.begin(), v.end(), a.mutable_data());
     return a;
 }
-template <class T>
-py::array_t<T> to_np2(const std::vector<T>& v, int rows, int cols) {
+template <class T, class A>
+py::array_t<T> to_np2(const std::vector<T, A>& v, int rows, int cols) {
     py::array_t<T> a({rows, cols});
     std::copy(v.begin(), v.begin() + (size_t)rows * cols, a.mutable_data());
     return a;
@@ -259,7 +259,8 @@ PYBIND11_MODULE(lightsim2grid_amd_cpp, m) {
         .def("compute_Vs", [](TimeSeries& ts, const darr& gen_p, const darr& sgen_p, const darr& load_p, const darr& load_q,
                               const carr& Vinit, int max_iter, double tol) {
             const int T = gen_p.ndim() == 2 ? (int)gen_p.shape(0) : (load_p.ndim() == 2 ? (int)load_p.shape(0) : 0);
-            RealVect gp = rvec(gen_p), sg = rvec(sgen_p), lp = rvec(load_p), lq = rvec(load_q);
+            auto view = [](const darr& a) { return RealView{a.data(), (size_t)a.size()}; };
+            const RealView gp = view(gen_p), sg = view(sgen_p), lp = view(load_p), lq = view(load_q);
             CplxVect v = cvec(Vinit);
             py::gil_scoped_release nogil;
             return ts.compute_Vs(T, gp, sg, lp, lq, v, max_iter, tol);
