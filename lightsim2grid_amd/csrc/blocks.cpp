@@ -77,6 +77,9 @@ Arms symbolic(int nb, std::vector<std::vector<int>>& low) {
 // The smallest tail worth a dense phase of its own.
 constexpr int kMinTail = 8;
 
+// Pairs that the 160 KB of a CU's LDS hold at most (one instance in FP32).
+constexpr int kMostUsed = 160 * 1024 / 8;
+
 }  // namespace
 
 bool has_block_form(const JPattern& J) { return J.rowpos.empty(); }
@@ -243,6 +246,21 @@ BlockPlan build_block_plan(const YbusPattern& Y, const JPattern& J, const std::v
         if (order == kByUse && places[a].tail != places[b].tail) return places[a].tail;
         return places[a].acc * places[b].size > places[b].acc * places[a].size;
     });
+    // Places that lie outside LDS in every launch: by the first column they serve, so that the blocks of a
+    // column, which products read together, share cache lines. 10 000-bus N-1 in FP32, a workgroup's factor
+    // levels 8.4 -> 6.9 ms and backward levels 2.5 -> 2.1. (By classes of use and column throughout, the FP64
+    // 2000-bus N-1 loses what that gains: 1.63 -> 1.80 ms.)
+    if (order == kByUse) {
+        auto column = [&](int p) {
+            const int id = places[p].ids[0];
+            if (id < 2 * nb) return id % nb;
+            const int q = id < vU ? id - vL : id - vU;
+            return (int)(std::upper_bound(A.cp.begin(), A.cp.end(), q) - A.cp.begin()) - 1;
+        };
+        size_t first = 0;
+        for (int pairs = next; first < po.size() && pairs < kMostUsed; ++first) pairs += places[po[first]].size;
+        std::stable_sort(po.begin() + first, po.end(), [&](int a, int b) { return column(a) < column(b); });
+    }
     P.second.assign(next, 0);
     P.fill_at = -1;
     for (int p : po) {
