@@ -473,7 +473,7 @@ __device__ __noinline__ double step_bus(double* V, VL Vl, bool v_lds, double* __
 }
 
 template <typename FT, int G, int NT, bool LEAN>
-__global__ void __launch_bounds__(NT) k_nr_block(const BArgs a) {
+__global__ void __launch_bounds__(NT, 4) k_nr_block(const BArgs a) {
     constexpr int kWaves = NT / 64;
     constexpr int nslot = NT / G;
     typedef FT ft2 __attribute__((ext_vector_type(2)));

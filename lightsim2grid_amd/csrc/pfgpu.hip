@@ -34,6 +34,7 @@
 #include <mutex>
 #include <stdexcept>
 #include <string>
+#include <tuple>
 #include <vector>
 
 #include "../../include/pfgpu.h"
@@ -1739,6 +1740,18 @@ int resident_blocks_of(const pfgpu_ctx* ctx, const void* fn, int NT, size_t lds)
     return per_cu * std::max(1, ctx->n_cu);
 }
 
+// The same from the last call of this shape (cached).
+int resident_blocks_cached(const pfgpu_ctx* ctx, const void* fn, int NT, size_t lds) {
+    static std::mutex mu;
+    static std::map<std::tuple<const void*, int, size_t, int>, int> cache;
+    std::lock_guard<std::mutex> lk(mu);
+    const auto key = std::make_tuple(fn, NT, lds, ctx->device);
+    const auto it = cache.find(key);
+    if (it != cache.end()) return it->second;
+    if (cache.size() >= 1024) cache.clear();
+    return cache[key] = resident_blocks_of(ctx, fn, NT, lds);
+}
+
 // Resident workgroups of a launch shape (occupancy of the kernel variant at its LDS size).
 int resident_blocks(const pfgpu_ctx* ctx, int fsize, int G, int NT, bool lean, size_t lds) {
     const void* fn;
@@ -1998,10 +2011,34 @@ struct BlockChoice {
     long long v_off;  // -1: V in global memory
 };
 
-// Launch heuristic: the largest G whose values and V fit entirely in LDS while keeping at least two
-// workgroups per CU; otherwise G = 1 with the most used pairs in LDS and the rest spilled. One workgroup
-// of 1024 lanes when its values take more than half of the LDS, else workgroups of 256.
+// Launch shape. G = 1 with the most used pairs in LDS and the rest spilled if the values of one instance and its
+// V do not fit; else the G that takes the least time by `rounds` of resident workgroups, a round taking about
+// 2.1 + G (a level's latency does not grow with G, its work does). One workgroup of 1024 lanes when its values
+// take more than half of the LDS, else workgroups of 256. Measured (MI355X, FP64, kernel time in us, G = 1, 2,
+// 4, 8): N-1 of 118 buses, 2000 instances: 316, 191, 164, 199; N-2 of 613 buses, 701: 473, 488, 409, 609; N-1
+// of 300 buses, 2000: 430, 491, 486, 908. Spilled at G > 1: 1200 buses, 2000: 1863, 1853, 2297.
+BlockChoice block_shape(const pfgpu_ctx* ctx, const pfgpu_grid::Block& b, int G, int fsize, int NT_req);
 BlockChoice choose_block(const pfgpu_ctx* ctx, const pfgpu_grid::Block& b, int ninst, int fsize, int G_req, int NT_req) {
+    if (G_req > 0) return block_shape(ctx, b, G_req, fsize, NT_req);
+    BlockChoice best = block_shape(ctx, b, 1, fsize, NT_req);
+    const long long ncu = std::max(1, ctx->n_cu);
+    if (ninst <= ncu || !best.lean || best.v_off < 0) return best;
+    double best_cost = 1e300;
+    for (int G = 1; G <= kMaxG; G *= 2) {
+        const BlockChoice c = G == 1 ? best : block_shape(ctx, b, G, fsize, NT_req);
+        if (c.G != G || !c.lean || c.v_off < 0) break;
+        const long long res = resident_blocks_cached(ctx, pfgpu_block::kernel(fsize, G, c.NT, true), c.NT, c.lds);
+        const long long groups = ((long long)ninst + G - 1) / G;
+        const double cost = (double)((groups + res - 1) / res) * (2.1 + G);
+        if (cost < best_cost) {
+            best_cost = cost;
+            best = c;
+        }
+    }
+    return best;
+}
+
+BlockChoice block_shape(const pfgpu_ctx* ctx, const pfgpu_grid::Block& b, int G, int fsize, int NT_req) {
     const pfgpu::BlockPlan& P = b.P;
     auto avail = [&](int G, int NT) -> size_t {
         const size_t fixed = pfgpu_block::state_bytes(G, NT) + 32;
@@ -2010,14 +2047,7 @@ BlockChoice choose_block(const pfgpu_ctx* ctx, const pfgpu_grid::Block& b, int n
     auto values = [&](int G) -> size_t { return (size_t)P.npairs * 2 * G * fsize; };
     const size_t fixed_pairs = (size_t)P.fixed_pairs;
     BlockChoice c{};
-    c.G = 1;
-    const long long ncu = std::max(1, ctx->n_cu);
-    if (G_req > 0) {
-        c.G = G_req;
-    } else {
-        for (int G = kMaxG; G >= 2; G >>= 1)
-            if (values(G) + (size_t)P.n * G * 16 <= avail(G, 1024) && (ninst + G - 1) / G >= 2 * ncu) { c.G = G; break; }
-    }
+    c.G = G;
     while (c.G > 1 && fixed_pairs * 2 * c.G * fsize > avail(c.G, 1024)) c.G >>= 1;
     c.NT = values(c.G) > avail(c.G, 1024) / 2 ? 1024 : 256;
     if (NT_req == 256 || NT_req == 1024) c.NT = NT_req;
