@@ -86,6 +86,7 @@ bool has_block_form(const JPattern& J) { return J.rowpos.empty(); }
 bool block_plan_fits(const BlockPlan& P) { return P.npairs < 1 << kBlkAddrBits; }
 
 BlockPlan build_block_plan(const YbusPattern& Y, const JPattern& J, const std::vector<int>& perm, BlockOrder order) {
+    if (order == kByLife) return by_life(build_block_plan(Y, J, perm, kByUse));
     BlockPlan P;
     const int n = Y.n, N = J.N;
     P.n = n;
@@ -210,12 +211,13 @@ BlockPlan build_block_plan(const YbusPattern& Y, const JPattern& J, const std::v
     // a block takes the place of one that was read for the last time before it is written (interval
     // colouring by size); places by decreasing accesses, so that a launch that cannot hold all of
     // them in LDS keeps the most used
-    struct Place { int size; long long acc; bool fill, tail; std::vector<int> ids; };  // fill: empty during the assembly
+    struct Place { int size; long long acc; bool fill, tail; int first; };  // fill: empty during the assembly
     auto in_tail = [&](int id) {
         if (id < 2 * nb) return id % nb >= k0;
         return (id < vU ? id - vL : id - vU) >= A.cp[k0];
     };
     std::vector<Place> places;
+    std::vector<int> place_of(nv, -1);
     auto colour = [&](std::vector<Life>& v, int size) {
         std::stable_sort(v.begin(), v.end(), [](const Life& a, const Life& b) { return a.t0 < b.t0; });
         using E = std::pair<int, int>;
@@ -227,9 +229,9 @@ BlockPlan build_block_plan(const YbusPattern& Y, const JPattern& J, const std::v
                 free.pop();
             } else {
                 p = (int)places.size();
-                places.push_back({size, 0, true, false, {}});
+                places.push_back({size, 0, true, false, x.id});
             }
-            places[p].ids.push_back(x.id);
+            place_of[x.id] = p;
             places[p].acc += x.acc;
             places[p].tail |= in_tail(x.id);
             if (x.t0 <= 0 || x.id >= nb && x.id < vL) places[p].fill = false;
@@ -242,37 +244,40 @@ BlockPlan build_block_plan(const YbusPattern& Y, const JPattern& J, const std::v
     std::vector<int> po(places.size());
     std::iota(po.begin(), po.end(), 0);
     std::stable_sort(po.begin(), po.end(), [&](int a, int b) {
-        if (order == kByLife && places[a].fill != places[b].fill) return places[b].fill;
-        if (order == kByUse && places[a].tail != places[b].tail) return places[a].tail;
+        if (places[a].tail != places[b].tail) return places[a].tail;
         return places[a].acc * places[b].size > places[b].acc * places[a].size;
     });
     // Places that lie outside LDS in every launch: by the first column they serve, so that the blocks of a
     // column, which products read together, share cache lines. 10 000-bus N-1 in FP32, a workgroup's factor
     // levels 8.4 -> 6.9 ms and backward levels 2.5 -> 2.1. (By classes of use and column throughout, the FP64
     // 2000-bus N-1 loses what that gains: 1.63 -> 1.80 ms.)
-    if (order == kByUse) {
+    {
         auto column = [&](int p) {
-            const int id = places[p].ids[0];
+            const int id = places[p].first;
             if (id < 2 * nb) return id % nb;
             const int q = id < vU ? id - vL : id - vU;
             return (int)(std::upper_bound(A.cp.begin(), A.cp.end(), q) - A.cp.begin()) - 1;
         };
         size_t first = 0;
         for (int pairs = next; first < po.size() && pairs < kMostUsed; ++first) pairs += places[po[first]].size;
-        std::stable_sort(po.begin() + first, po.end(), [&](int a, int b) { return column(a) < column(b); });
+        std::vector<int> col(places.size());
+        for (size_t i = first; i < po.size(); ++i) col[po[i]] = column(po[i]);
+        std::stable_sort(po.begin() + first, po.end(), [&](int a, int b) { return col[a] < col[b]; });
     }
     P.second.assign(next, 0);
-    P.fill_at = -1;
+    std::vector<int> at_of(places.size());
     for (int p : po) {
-        if (order == kByLife && places[p].fill && P.fill_at < 0) P.fill_at = next;
-        for (int id : places[p].ids) addr[id] = next;
+        P.places.push_back({next, places[p].size, places[p].acc, places[p].fill});
+        at_of[p] = next;
         next += places[p].size;
         if (places[p].tail) P.fixed_pairs = next;
         P.second.push_back(0);
         if (places[p].size == 2) P.second.push_back(1);
     }
+    for (int id = 0; id < nv; ++id)
+        if (place_of[id] >= 0) addr[id] = at_of[place_of[id]];
     P.second.resize(next + 2, 0);
-    if (P.fill_at < 0) P.fill_at = next;
+    P.fill_at = next;
     P.npairs = next + 1;  // a one-pair block's second pair is read (and not used)
 
     // --- target words -----------------------------------------------------------------------------
@@ -410,6 +415,54 @@ BlockPlan build_block_plan(const YbusPattern& Y, const JPattern& J, const std::v
             P.jd_jidx.insert(P.jd_jidx.end(), &jx[4 * (size_t)q], &jx[4 * (size_t)q] + 4);
         }
     }
+    return P;
+}
+
+// The same places in another order: nothing but the pairs' names changes.
+BlockPlan by_life(BlockPlan P) {
+    std::vector<BlockPlan::Place> to = P.places;
+    std::stable_sort(to.begin(), to.end(), [](const BlockPlan::Place& a, const BlockPlan::Place& b) {
+        if (a.fill != b.fill) return b.fill;
+        return a.acc * b.size > b.acc * a.size;
+    });
+    std::vector<int> name(P.npairs + 1, 0);
+    int next = 2;  // after the zeros
+    for (int q : {0, 1}) name[q] = q;
+    P.second.assign(next, 0);
+    P.fill_at = -1;
+    for (auto& p : to) {
+        if (p.fill && P.fill_at < 0) P.fill_at = next;
+        for (int k = 0; k < p.size; ++k) {
+            name[p.at + k] = next++;
+            P.second.push_back(k == 1);
+        }
+        p.at = next - p.size;
+    }
+    name[next] = next;
+    P.second.resize(next + 2, 0);
+    if (P.fill_at < 0) P.fill_at = next;
+    P.fixed_pairs = P.npairs;
+    P.places = std::move(to);
+    auto word = [&](int& w) {
+        if (w != -1) w = (w & ~kBlkAddrMask) | name[w & kBlkAddrMask];
+    };
+    auto pair = [&](int& q) { q = name[q]; };
+    auto each = [](std::vector<int>& v, size_t from, size_t step, auto f) {
+        for (size_t i = from; i < v.size(); i += step) f(v[i]);
+    };
+    each(P.bus_y, 0, 1, word);
+    if (P.slack_x >= 0) pair(P.slack_x);
+    each(P.tail_src, 0, 1, [&](int& x) { x = 2 * name[x >> 1] + (x & 1); });
+    each(P.rows, 1, 4, word);
+    each(P.rows, 3, 4, word);
+    each(P.jd, 1, 2, word);
+    each(P.jc_dst, 0, 1, word);
+    each(P.tasks, 0, 3, word);
+    each(P.prods, 0, 1, pair);
+    each(P.btasks, 0, 4, word);
+    each(P.btasks, 3, 4, pair);
+    each(P.bprods, 0, 3, pair);
+    each(P.bprods, 1, 3, pair);
     return P;
 }
 

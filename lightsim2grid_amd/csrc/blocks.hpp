@@ -56,6 +56,14 @@ struct BlockPlan {
     // where the dense phase finds its matrix: per entry, row-major [m][m + 1], the number's place (2 pair +
     // component); column m is the right-hand side, which receives the solution
     std::vector<int> tail_src;
+    // where blocks are stored, in the order of the pairs: first pair, pairs, accesses, whether it is empty while J
+    // is assembled
+    struct Place {
+        int at, size;
+        long long acc;
+        bool fill;
+    };
+    std::vector<Place> places;
     std::vector<char> second;   // per pair: the second one of a block (npairs + 1 entries)
     // Assembly of F and J by Ybus rows (the buses with unknowns), longest first: per row {bus, its pair
     // word (bus_y), CSC position and target word of the diagonal entry}; the other entries as jagged
@@ -80,6 +88,8 @@ bool block_plan_fits(const BlockPlan& P);
 enum BlockOrder { kByUse = 0, kByLife = 1 };
 // perm: the bus-block elimination order of J (column_order)
 BlockPlan build_block_plan(const YbusPattern& Y, const JPattern& J, const std::vector<int>& perm, BlockOrder order = kByUse);
+// a plan in order kByUse, in order kByLife
+BlockPlan by_life(BlockPlan P);
 
 // Unit streams of the block plan for one launch shape: G interleaved instances, `waves` waves per
 // workgroup, values of fsize bytes, the first nlds pairs in LDS. Each wave has a stream of its own of

@@ -2104,7 +2104,7 @@ pfgpu_grid::Block::Lanes& block_lanes(pfgpu_grid::Block& b, const BlockChoice& c
     return *slot;
 }
 
-std::unique_ptr<pfgpu_grid::Block> upload_blocks(const pfgpu_grid* g, const std::vector<int>& perm, pfgpu::BlockOrder order);
+std::unique_ptr<pfgpu_grid::Block> upload_blocks(const pfgpu_grid* g, pfgpu::BlockPlan plan);
 
 // One NR launch on the block plan; as launch_pass otherwise.
 void launch_block(pfgpu_ctx* ctx, pfgpu_grid* gr, const SolveArgs& q, int precision, int G_req, int NT_req, int nunits,
@@ -2113,7 +2113,7 @@ void launch_block(pfgpu_ctx* ctx, pfgpu_grid* gr, const SolveArgs& q, int precis
     BlockChoice c = choose_block(ctx, *gr->blk, nunits, fsize, G_req, NT_req);
     pfgpu_grid::Block* use = gr->blk.get();
     if (c.lean && c.v_off < 0) {  // V does not fit beside the values: over some of them?
-        if (!gr->blk_life && !fx) gr->blk_life = upload_blocks(gr, pfgpu::column_order(gr->J), pfgpu::kByLife);
+        if (!gr->blk_life && !fx) gr->blk_life = upload_blocks(gr, pfgpu::by_life(gr->blk->P));
         if (gr->blk_life) {
             const BlockChoice cl = choose_block(ctx, *gr->blk_life, nunits, fsize, c.G, c.NT);
             if (cl.v_off >= 0) {
@@ -2793,9 +2793,9 @@ void upload_rows(pfgpu_grid* g) {
 }
 
 // A block plan and its tables on the device.
-std::unique_ptr<pfgpu_grid::Block> upload_blocks(const pfgpu_grid* g, const std::vector<int>& perm, pfgpu::BlockOrder order) {
+std::unique_ptr<pfgpu_grid::Block> upload_blocks(const pfgpu_grid* g, pfgpu::BlockPlan plan) {
     auto b = std::make_unique<pfgpu_grid::Block>();
-    b->P = pfgpu::build_block_plan(g->Y, g->J, perm, order);
+    b->P = std::move(plan);
     const pfgpu::BlockPlan& B = b->P;
     if (!pfgpu::block_plan_fits(B)) return nullptr;
     Tables tab;
@@ -2823,7 +2823,7 @@ std::unique_ptr<pfgpu_grid::Block> upload_blocks(const pfgpu_grid* g, const std:
 // target words can name keeps the scalar plan.)
 void build_blocks(pfgpu_grid* g) {
     const std::vector<int> perm = pfgpu::column_order(g->J);
-    g->blk = upload_blocks(g, perm, pfgpu::kByUse);
+    g->blk = upload_blocks(g, pfgpu::build_block_plan(g->Y, g->J, perm));
     if (!g->blk) return;
     const pfgpu::BlockPlan& B = g->blk->P;
     pfgpu::DevicePlan& P = g->P;
