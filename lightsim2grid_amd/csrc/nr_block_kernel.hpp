@@ -200,8 +200,13 @@ struct Values {
             if (two) Pl[(q + 1) * G + g] = p1;
         } else {
             ft2* const p = Pg + (size_t)(q - nlds) * G + g;
-            p[0] = p0;
-            if (two) p[G] = p1;
+            if (G == 1 && two) {  // one store: scattered lanes take a cycle each
+                typedef FT ft4 __attribute__((ext_vector_type(4), aligned(2 * sizeof(FT))));
+                *(ft4*)p = ft4{p0.x, p0.y, p1.x, p1.y};
+            } else {
+                p[0] = p0;
+                if (two) p[G] = p1;
+            }
         }
     }
     // writes a block that is no pivot
