@@ -2022,7 +2022,19 @@ BlockChoice choose_block(const pfgpu_ctx* ctx, const pfgpu_grid::Block& b, int n
     if (G_req > 0) return block_shape(ctx, b, G_req, fsize, NT_req);
     BlockChoice best = block_shape(ctx, b, 1, fsize, NT_req);
     const long long ncu = std::max(1, ctx->n_cu);
-    if (ninst <= ncu || !best.lean || best.v_off < 0) return best;
+    if (ninst <= ncu) return best;
+    // FP64 values of five times the LDS and more: most operands are read from memory, where four instances side
+    // by side make whole cache lines. Of the 10 000-bus grid a round of G = 1, 2, 4 takes 4.4, 7.1, 11.4 ms
+    // (G = 1 and 4: 9692 outages 166, 108 ms; 2000 34.6, 23.4; 600 11.2, 13.1); of the 3000-bus grid, 2.6 times the
+    // LDS, 0.75, 1.6, 2.7. In FP32 (10 000 buses) 2.2, 5.4, 9.1.
+    if (fsize == 8 && (size_t)b.P.npairs * 16 >= 5 * (size_t)ctx->lds_max) {
+        const double one = (double)ninst / (double)ncu;
+        if (std::max(one / 4, 1.0) * 2.6 < one) {
+            const BlockChoice c = block_shape(ctx, b, 4, fsize, NT_req);
+            if (c.G == 4) return c;
+        }
+    }
+    if (!best.lean || best.v_off < 0) return best;
     double best_cost = 1e300;
     for (int G = 1; G <= kMaxG; G *= 2) {
         const BlockChoice c = G == 1 ? best : block_shape(ctx, b, G, fsize, NT_req);
@@ -2111,6 +2123,11 @@ void launch_block(pfgpu_ctx* ctx, pfgpu_grid* gr, const SolveArgs& q, int precis
                   const int* imap, const AuxLayout& AL, bool fresh, pfgpu_stats* st, const FixedScratch* fx) {
     const int fsize = precision == PFGPU_FP64 ? 8 : 4;
     BlockChoice c = choose_block(ctx, *gr->blk, nunits, fsize, G_req, NT_req);
+    auto rows_of = [&](const BlockChoice& x) {  // workspace of a workgroup
+        return (size_t)x.G * gr->P.n * 16 + (size_t)x.nspill * 2 * x.G * fsize;
+    };
+    if (fx && G_req == 0 && c.G > 1 && rows_of(c) + 1024 > fx->ws_bytes)
+        c = block_shape(ctx, *gr->blk, 1, fsize, NT_req);
     pfgpu_grid::Block* use = gr->blk.get();
     if (c.lean && c.v_off < 0) {  // V does not fit beside the values: over some of them?
         if (!gr->blk_life && !fx) gr->blk_life = upload_blocks(gr, pfgpu::by_life(gr->blk->P));
@@ -2137,7 +2154,7 @@ void launch_block(pfgpu_ctx* ctx, pfgpu_grid* gr, const SolveArgs& q, int precis
     const size_t gather_bytes = gather ? o_yrow + align_up((size_t)std::max(nrow, 1) * 16) : 0;
     if (fx) {
         // workgroups whose rows fit the fixed workspace (4 * 256 bytes covers the roundings)
-        const size_t per_block = (size_t)c.G * n * 16 + (size_t)c.nspill * 2 * c.G * fsize;
+        const size_t per_block = rows_of(c);
         const size_t room = fx->ws_bytes > gather_bytes + 1024 ? fx->ws_bytes - gather_bytes - 1024 : 0;
         const long long cap = per_block ? (long long)(room / per_block) : nres;
         if (cap < 1) throw ApiError(PFGPU_E_BUDGET, "the grid's per-workgroup rows do not fit the fixed scratch");

@@ -111,3 +111,28 @@ def test_shortest_time_launch_with_and_without_a_block_form(gpu_ctx, oracle_mod,
         assert r["status"][0] == 0 and r["iters"][0] == o.get_nb_iter()
         assert np.max(np.abs(r["V"][0] - o.get_V())) <= 1e-8
     assert r["stats"]["workgroups"] > 1  # the wide kernel's
+
+
+@pytest.mark.parametrize("n,rows,prec,more", [(60, 600, 0, False), (118, 1100, 0, True), (118, 2000, 2, True),
+                                              (10000, 800, 0, True), (10000, 600, 0, False)])
+def test_default_launch_shape_equals_one_instance_per_workgroup(gpu_ctx, n, rows, prec, more):
+    """The shape that a launch takes by itself (`more`: several instances per workgroup) against G = 1: equal
+    statuses, FP64 equal iterations and |dV| <= 1e-9, FP32 the bound of the FP32 form."""
+    from lightsim2grid_amd import abi, gridgen
+    _say("default shape", n, rows, prec)
+    g = gridgen.make(f"case{n}_synth") if n in (118, 10000) else gridgen.generate(n, n + n // 3, n // 4, 3, loading=0.3)
+    d = g.solver_inputs()
+    gr = abi.Grid(gpu_ctx, d["Ybus"], d["slack_ids"], d["slack_weights"], d["pv"], d["pq"])
+    Yx = gr.ybus_values(d["Ybus"])
+    base = gr.solve(Yx, d["Sbus"], d["V0"], 10, 1e-8)
+    assert base["status"][0] == 0
+    lines = np.nonzero(~gridgen.bridges(g))[0]
+    deltas = g.ybus_deltas([[int(lines[k % len(lines)])] for k in range(rows)])
+    r0, r1 = (gr.solve(Yx, d["Sbus"], base["V"][0], 10, 1e-8, precision=prec, deltas=deltas, instances_per_wg=G)
+              for G in (0, 1))
+    assert (r0["stats"]["instances_per_wg"] > 1) == more
+    assert np.array_equal(r0["status"], r1["status"])
+    ok = r1["status"] == 0
+    if prec == abi.FP64:
+        assert np.array_equal(r0["iters"][ok], r1["iters"][ok])
+    assert np.max(np.abs(r0["V"][ok] - r1["V"][ok])) <= (1e-9 if prec == abi.FP64 else 5e-8)
