@@ -496,36 +496,35 @@ std::vector<Chunk> deal_level(const std::vector<int>& np, int G, int waves) {
     std::vector<int> ord(nt);
     std::iota(ord.begin(), ord.end(), 0);
     std::stable_sort(ord.begin(), ord.end(), [&](int a, int b) { return np[a] > np[b]; });
-    auto deal = [&](int n) {
-        std::vector<Chunk> out;
-        for (size_t i = 0; i < ord.size();) {
-            Chunk c;
-            c.lt = std::min(tmax, log2_up(std::max(1, (np[ord[i]] + n - 1) / n)));
-            c.n = std::max(1, (np[ord[i]] + (1 << c.lt) - 1) >> c.lt);
-            for (int k = 0; k < width >> c.lt && i < ord.size(); ++k) c.tasks.push_back(ord[i++]);
-            out.push_back(std::move(c));
+    auto deal = [&](int n, auto chunk) {  // chunk(lt, units, first task, tasks)
+        for (int i = 0; i < nt;) {
+            const int p = np[ord[i]], lt = std::min(tmax, log2_up(std::max(1, (p + n - 1) / n)));
+            const int m = std::min(width >> lt, nt - i);
+            chunk(lt, std::max(1, (p + (1 << lt) - 1) >> lt), i, m);
+            i += m;
         }
-        return out;
     };
-    std::vector<Chunk> best;
+    int best = 1;
     double best_cost = 1e300;
     for (int n = (maxnp + (1 << tmax) - 1) >> tmax; n <= maxnp; n = n < 16 ? n + 1 : n + n / 8) {
-        std::vector<Chunk> c = deal(std::max(1, n));
-        std::vector<double> simd(4, 0.0);
-        double chain = 0;
-        for (size_t i = 0; i < c.size(); ++i) {
-            const double issue = 4.5 * (28.0 * c[i].n + 5.0 * c[i].lt + 50.0);
-            simd[i % waves % 4] += issue;
-            chain = std::max(chain, 300.0 + 40.0 * c[i].n + 25.0 * c[i].lt);
-        }
-        const double issue = *std::max_element(simd.begin(), simd.end());
+        double simd[4] = {0, 0, 0, 0}, chain = 0;
+        int i = 0;
+        deal(std::max(1, n), [&](int lt, int units, int, int) {
+            simd[i++ % waves % 4] += 4.5 * (28.0 * units + 5.0 * lt + 50.0);
+            chain = std::max(chain, 300.0 + 40.0 * units + 25.0 * lt);
+        });
+        const double issue = *std::max_element(simd, simd + 4);
         const double cost = std::max(chain, issue) + 0.1 * issue;
         if (cost < best_cost - 1e-9) {
             best_cost = cost;
-            best = std::move(c);
+            best = std::max(1, n);
         }
     }
-    return best;
+    std::vector<Chunk> out;
+    deal(best, [&](int lt, int units, int first, int m) {
+        out.push_back({lt, units, std::vector<int>(ord.begin() + first, ord.begin() + first + m)});
+    });
+    return out;
 }
 
 // Lays the levels out: emit(task, product in the task or -1, last unit, unit) fills a lane's unit, which
@@ -551,7 +550,8 @@ void lay_levels(const std::vector<int>& lvl, int G, int waves, NProds nprods, Em
             for (int u = 0; u < c.n; ++u) {
                 const bool end = u == c.n - 1;
                 const size_t p = st.size();
-                for (int k = 0; k < 64; ++k) st.insert(st.end(), pad, pad + 4);
+                st.resize(p + 256);
+                for (int k = 0; k < 64; ++k) std::copy(pad, pad + 4, &st[p + 4 * k]);
                 for (size_t k = 0; k < c.tasks.size(); ++k)
                     for (int tp = 0; tp < T; ++tp) {
                         const int i = c.tasks[k], pi = u * T + tp;
@@ -571,6 +571,11 @@ void lay_levels(const std::vector<int>& lvl, int G, int waves, NProds nprods, Em
     at.assign(waves, 0);
     for (int w = 0; w < waves; ++w) {
         at[w] = (int)(out.size() / 256);
+        if (w == 0) {
+            size_t all = 0;
+            for (const auto& s : ws) all += s.size() + 512 * kBlkAhead;
+            out.reserve(all);
+        }
         out.insert(out.end(), ws[w].begin(), ws[w].end());
         for (int k = 0; k < 64 * 2 * kBlkAhead; ++k) out.insert(out.end(), pad, pad + 4);
     }
