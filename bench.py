@@ -385,7 +385,7 @@ def large_grid_run(with_cpu: bool, nthreads: int, n_out: int = 5000, n_snap: int
                 lat.append(r["stats"]["kernel_s"])
             out[nm][key] = 1e3 * float(np.median(lat))
             if G == 0:
-                out[nm]["single_solve_launch"] = "wide" if r["stats"]["instances_per_wg"] == -1 else "batched"
+                out[nm]["single_solve_launch"] = "single instance" if r["stats"]["instances_per_wg"] == -1 else "batched"
     if with_cpu:
         from oracle import oracle
         k = 16 * nthreads
@@ -545,7 +545,7 @@ def single_solves(name: str, reps: int = 5) -> dict:
             for _ in range(reps):
                 r = gr.solve(Yx, d["Sbus"], d["V0"], 10, 1e-8, precision=prec, instances_per_wg=G)
                 ms.append(1e3 * r["stats"]["kernel_s"])
-            out[f"{nm}_{key}"] = {"launch": "wide" if r["stats"]["instances_per_wg"] == -1 else "batched",
+            out[f"{nm}_{key}"] = {"launch": "single instance" if r["stats"]["instances_per_wg"] == -1 else "batched",
                                   "iters": int(r["iters"][0]), "status": int(r["status"][0]),
                                   "kernel_ms": ms}
     gr.close()
@@ -731,7 +731,7 @@ def main():
                      "traffic": measured_traffic("fp32") if args.grid == "case2000_synth" else None,
                      "traffic_source": "profiles/k_nr_case2000_n1_hbm_traffic.md",
                      "bytes_per_launch": r32["bytes_per_launch"], "priced_on": "converged solves",
-                     "kernel": "k_nr<float,G,block,lean>", "kernel_ms": r32["kernel_ms"]},
+                     "kernel": "k_nr_block<float,G,block,lean>", "kernel_ms": r32["kernel_ms"]},
         "cpu_baseline": cpu,
         "parity": par,
         "fp64_form": {"value": r64["solves_per_s"], "ms_per_step": r64["ms_per_step"], "kernel_ms": r64["kernel_ms"],

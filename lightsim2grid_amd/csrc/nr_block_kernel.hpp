@@ -17,8 +17,8 @@
 // of unknowns shorten the chain (2000 buses: 33 + 33 levels for 53 + 53) and cut the products 4.8 times. The
 // units of a wave are a stream of its own with byte offsets and wave-uniform control, so a product takes no
 // decoding, a team no selects and no level a table look-up. Against the scalar kernel (k_nr) it took the
-// 2000-bus N-1 sweep (2128 outages) from 3.65 to 2.04 ms with FP32 and from 8.2 to 4.5 ms with FP64 factors,
-// 1500 outages of 10 000 buses from 46.9 to 17.7 ms, 701 N-2 outages of 613 buses from 0.57 to 0.42 ms.
+// 2000-bus N-1 sweep (2128 outages) from 3.65 to 1.89 ms with FP32 and from 8.2 to 3.8 ms with FP64 factors,
+// 1500 outages of 10 000 buses from 46.9 to 14.3 ms, 701 N-2 outages of 613 buses from 0.57 to 0.41 ms.
 #pragma once
 
 #include "nr_block.hpp"

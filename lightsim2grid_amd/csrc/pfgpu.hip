@@ -2015,8 +2015,8 @@ struct BlockChoice {
 // V do not fit; else the G that takes the least time by `rounds` of resident workgroups, a round taking about
 // 2.1 + G (a level's latency does not grow with G, its work does). One workgroup of 1024 lanes when its values
 // take more than half of the LDS, else workgroups of 256. Measured (MI355X, FP64, kernel time in us, G = 1, 2,
-// 4, 8): N-1 of 118 buses, 2000 instances: 316, 191, 164, 199; N-2 of 613 buses, 701: 473, 488, 409, 609; N-1
-// of 300 buses, 2000: 430, 491, 486, 908. Spilled at G > 1: 1200 buses, 2000: 1863, 1853, 2297.
+// 4, 8): N-1 of 118 buses, 2000 instances: 213, 169, 193, 198; of 300 buses, 2000: 363, 519, 481, 894; 40 buses,
+// 1500: 168, 169, 156, 183. Spilled at G > 1: 613 buses, 701: 415, 481, 409, 611; 1200, 2000: 1863, 1853, 2297.
 BlockChoice block_shape(const pfgpu_ctx* ctx, const pfgpu_grid::Block& b, int G, int fsize, int NT_req);
 BlockChoice choose_block(const pfgpu_ctx* ctx, const pfgpu_grid::Block& b, int ninst, int fsize, int G_req, int NT_req) {
     if (G_req > 0) return block_shape(ctx, b, G_req, fsize, NT_req);
@@ -2229,7 +2229,7 @@ void launch_pass(pfgpu_ctx* ctx, pfgpu_grid* gr, const SolveArgs& q, int precisi
     if (wide_wanted(gr, q, G_req, nunits, fx)) {
         // A plan with a block form takes one workgroup per instance here too: the grid-wide barrier of every
         // level costs more than the other workgroups' lanes give. One solve from V0 in FP64 (FP32), ms:
-        // 2000 buses 0.68 against 2.3 wide, 5000 1.3 (0.9) against 3.4, 10 000 3.9 (2.8) against 8.2 (7.7),
+        // 2000 buses 0.51 against 2.3 wide, 5000 1.3 (0.9) against 3.4, 10 000 4.0 (2.8) against 8.2 (7.7),
         // 20 000 9.8 (7.3) against 25 (22), 40 000 24 (18) against 51 (45).
         if (gr->blk) {
             launch_block(ctx, gr, q, precision, 1, 1024, nunits, imap, AL, fresh, st, fx);
