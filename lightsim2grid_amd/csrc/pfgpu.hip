@@ -1115,10 +1115,41 @@ __global__ void k_gather_y(const double* __restrict__ Y, const int2* __restrict_
     }
 }
 
-// The same for the block plan: off-diagonal entries in jagged-diagonal order, then the rows' diagonals.
-__global__ void k_gather_rows(const double* __restrict__ Y, const int* __restrict__ jd_pos, int nent,
-                              const int4* __restrict__ rows, int nrow, double* __restrict__ Yjd, double* __restrict__ Yrow) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+// The first kernel of a solve launch: zeroes the NR kernel's work-queue counter and, unless
+// the voltages are solved in place, writes the initial V of every launch instance (its first
+// row: the chain head in chain mode) from V0 (one row per instance, or one shared row).
+__device__ __forceinline__ void init_v(const double* V0, long long v0_stride, double* V, int n, int ninst, const int* imap,
+                                       int chain, int* queue, unsigned long long* phase, int copy, int nblocks) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) *queue = 0;
+    if (blockIdx.x == 0 && threadIdx.x < 8 && phase) phase[threadIdx.x] = 0;
+    if (!copy) return;
+    const long long total = (long long)ninst * n;
+    for (long long k = blockIdx.x * (long long)blockDim.x + threadIdx.x; k < total; k += (long long)nblocks * blockDim.x) {
+        const long long i = k / n;
+        const int b = (int)(k - i * n);
+        const long long oi = imap ? (long long)imap[i] : i;
+        const long long r = oi * chain;
+        V[2 * (r * n + b)] = V0[oi * v0_stride + 2 * b];
+        V[2 * (r * n + b) + 1] = V0[oi * v0_stride + 2 * b + 1];
+    }
+}
+__global__ void k_init_v(const double* V0, long long v0_stride, double* V, int n, int ninst, const int* imap,
+                         int chain, int* queue, unsigned long long* phase, int copy) {
+    init_v(V0, v0_stride, V, n, ninst, imap, chain, queue, phase, copy, gridDim.x);
+}
+
+// The same for the block plan, in its first `nblocks` workgroups; the others gather a shared Ybus: its
+// off-diagonal entries in jagged-diagonal order, then the rows' diagonals. One launch: a small solve is a few
+// tens of microseconds, and a kernel of its own for each costs it about 5.
+__global__ void k_begin(const double* V0, long long v0_stride, double* V, int n, int ninst, const int* imap, int chain,
+                        int* queue, unsigned long long* phase, int copy, int nblocks, const double* __restrict__ Y,
+                        const int* __restrict__ jd_pos, int nent, const int4* __restrict__ rows, int nrow,
+                        double* __restrict__ Yjd, double* __restrict__ Yrow) {
+    if ((int)blockIdx.x < nblocks) {
+        init_v(V0, v0_stride, V, n, ninst, imap, chain, queue, phase, copy, nblocks);
+        return;
+    }
+    const int i = (blockIdx.x - nblocks) * blockDim.x + threadIdx.x;
     if (i < nent) {
         const int p = jd_pos[i];
         Yjd[2 * i] = Y[2 * p];
@@ -1127,26 +1158,6 @@ __global__ void k_gather_rows(const double* __restrict__ Y, const int* __restric
         const int r = i - nent, p = rows[r].z;
         Yrow[2 * r] = Y[2 * p];
         Yrow[2 * r + 1] = Y[2 * p + 1];
-    }
-}
-
-// The first kernel of a solve launch: zeroes the NR kernel's work-queue counter and, unless
-// the voltages are solved in place, writes the initial V of every launch instance (its first
-// row: the chain head in chain mode) from V0 (one row per instance, or one shared row).
-__global__ void k_init_v(const double* V0, long long v0_stride, double* V, int n, int ninst, const int* imap,
-                         int chain, int* queue, unsigned long long* phase, int copy) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) *queue = 0;
-    if (blockIdx.x == 0 && threadIdx.x < 8 && phase) phase[threadIdx.x] = 0;
-    if (!copy) return;
-    const long long total = (long long)ninst * n;
-    for (long long k = blockIdx.x * (long long)blockDim.x + threadIdx.x; k < total;
-         k += (long long)gridDim.x * blockDim.x) {
-        const long long i = k / n;
-        const int b = (int)(k - i * n);
-        const long long oi = imap ? (long long)imap[i] : i;
-        const long long r = oi * chain;
-        V[2 * (r * n + b)] = V0[oi * v0_stride + 2 * b];
-        V[2 * (r * n + b) + 1] = V0[oi * v0_stride + 2 * b + 1];
     }
 }
 
@@ -1438,7 +1449,7 @@ struct pfgpu_grid {
         DevBuf<int> f_lvl, b_lvl, f_team, b_team, tasks, pairs, btasks, bpairs;
         int blocks = 0;
     } wide;
-    // Launch sequences (k_init_v, k_gather_y, k_nr) captured as HIP graphs, by the exact launch
+    // Launch sequences (k_begin or k_init_v and k_gather_y, the NR kernel) captured as HIP graphs, by the exact launch
     // arguments: a sequence seen a second time is captured, and replayed from then on.
     struct GraphEntry {
         std::vector<unsigned char> key;
@@ -1723,6 +1734,11 @@ struct SolveArgs {
     bool* out_done = nullptr;
 };
 
+// Workgroups that write the initial V.
+int init_blocks(bool copy, long long nunits, int n) {
+    return copy ? (int)std::min<long long>(std::max<long long>((nunits * n + 255) / 256, 1), 1024) : 1;
+}
+
 // What the caller of a launch wants on the stream before the wait for it.
 void run_before_sync(pfgpu_ctx* ctx) {
     if (!ctx->before_sync) return;
@@ -1883,7 +1899,7 @@ void launch_wide(pfgpu_ctx* ctx, pfgpu_grid* gr, const SolveArgs& q, int precisi
     a.red = reinterpret_cast<double*>(ws + o_red); a.ctl = reinterpret_cast<int*>(ws + o_ctl);
     a.bar = reinterpret_cast<unsigned int*>(ws + o_bar);
     HIP_OK(hipEventRecord(ctx->ev0, stream));
-    hipLaunchKernelGGL(k_init_v, dim3(copy ? 1024 : 1), dim3(256), 0, stream, q.V0, (long long)q.v0_stride * 2, q.V, n,
+    hipLaunchKernelGGL(k_init_v, dim3(init_blocks(copy, nunits, n)), dim3(256), 0, stream, q.V0, (long long)q.v0_stride * 2, q.V, n,
                        nunits, imap, q.chain, reinterpret_cast<int*>(aux + AL.o_queue), nullptr, copy ? 1 : 0);
     HIP_OK(hipGetLastError());
     HIP_OK(pfgpu_wide::launch(a, fp32, lds, stream));
@@ -2204,14 +2220,11 @@ void launch_block(pfgpu_ctx* ctx, pfgpu_grid* gr, const SolveArgs& q, int precis
     a.Jx_last = q.Jx_last; a.jx_row = q.jx_row; a.imap = imap; a.nrows = q.nrows; a.phase_t = phase; a.queue = queue;
     a.ngroups = ngroups;
     auto issue = [&]() {
-        hipLaunchKernelGGL(k_init_v, dim3(copy ? 1024 : 1), dim3(256), 0, stream, q.V0, (long long)q.v0_stride * 2, q.V,
-                           n, nunits, imap, q.chain, queue, phase, copy ? 1 : 0);
+        const int nb = init_blocks(copy, nunits, n), ng = gather ? (nent + nrow + 255) / 256 : 0;
+        hipLaunchKernelGGL(k_begin, dim3(nb + ng), dim3(256), 0, stream, q.V0, (long long)q.v0_stride * 2, q.V, n, nunits,
+                           imap, q.chain, queue, phase, copy ? 1 : 0, nb, q.Yx, b.jd_pos.p, nent, a.rows, nrow,
+                           reinterpret_cast<double*>(ws + o_y), reinterpret_cast<double*>(ws + o_y + o_yrow));
         HIP_OK(hipGetLastError());
-        if (gather) {
-            hipLaunchKernelGGL(k_gather_rows, dim3((nent + nrow + 255) / 256), dim3(256), 0, stream, q.Yx, b.jd_pos.p, nent,
-                               a.rows, nrow, reinterpret_cast<double*>(ws + o_y), reinterpret_cast<double*>(ws + o_y + o_yrow));
-            HIP_OK(hipGetLastError());
-        }
         pfgpu_block::launch(a, fsize, c.G, c.NT, c.lean, nres, c.lds, stream);
     };
     run_sequence(ctx, gr, sequence_key(&a, sizeof(a), q, copy, nres, c.G, c.NT, c.lean, fsize, gather, c.lds), issue, fx,
@@ -2338,7 +2351,7 @@ void launch_pass(pfgpu_ctx* ctx, pfgpu_grid* gr, const SolveArgs& q, int precisi
     if (gr->dc) a.max_iter = 1;
     const int nell = gr->ell_w * n, nye = (int)P.ye_pos.size();
     auto issue = [&]() {
-        hipLaunchKernelGGL(k_init_v, dim3(copy ? 1024 : 1), dim3(256), 0, stream, q.V0, (long long)q.v0_stride * 2, q.V,
+        hipLaunchKernelGGL(k_init_v, dim3(init_blocks(copy, nunits, n)), dim3(256), 0, stream, q.V0, (long long)q.v0_stride * 2, q.V,
                            n, nunits, imap, q.chain, queue, phase, copy ? 1 : 0);
         HIP_OK(hipGetLastError());
         if (gather) {
