@@ -117,10 +117,15 @@ BlockPlan build_block_plan(const YbusPattern& Y, const JPattern& J, const std::v
     }
     // value ids: D(k) = k, y(k) = nb + k, L = 2 nb + q, U = 2 nb + na + q
     const int vL = 2 * nb, vU = 2 * nb + na, nv = 2 * nb + 2 * na;
-    auto id_of = [&](int a, int b) {
+    auto find_block = [&](int a, int b) {  // -1: not in the symmetrised pattern
         if (a == b) return a;
-        if (a > b) return vL + find_in(A.ci, A.cp[b], A.cp[b + 1], a);
-        return vU + find_in(A.ci, A.cp[a], A.cp[a + 1], b);
+        const int k = std::min(a, b), q = find_in(A.ci, A.cp[k], A.cp[k + 1], std::max(a, b));
+        return q < 0 ? -1 : (a > b ? vL : vU) + q;
+    };
+    auto id_of = [&](int a, int b) {
+        const int id = find_block(a, b);
+        if (id < 0) throw std::logic_error("pfgpu: a block outside the factor's pattern");
+        return id;
     };
     struct Prod { int t, l, u, d; };
     std::vector<Prod> pr;
@@ -347,8 +352,9 @@ BlockPlan build_block_plan(const YbusPattern& Y, const JPattern& J, const std::v
         for (int r = 0; r < B.w[a]; ++r) {
             for (int b = k0; b < nb; ++b)
                 for (int c = 0; c < B.w[b]; ++c) {
-                    const int id = id_of(a, b);
-                    const bool has = a == b || (a < b ? hasU[id - vU] : hasL[id - vL]);
+                    // the top chain of the elimination tree need not be dense
+                    const int id = find_block(a, b);
+                    const bool has = a == b || (id >= 0 && (a < b ? hasU[id - vU] : hasL[id - vL]));
                     P.tail_src.push_back(!has ? 2 * P.zpair : a < b ? 2 * (addr[id] + c) + r : 2 * (addr[id] + r) + c);
                 }
             P.tail_src.push_back(2 * addr[nb + a] + r);
