@@ -760,10 +760,8 @@ __global__ void __launch_bounds__(NT, 4) k_nr_block(const BArgs a) {
         }
         tmark(1);
         // ---- dense tail ---------------------------------------------------------------------------
-        if (m > 0) {
-            tail_by_waves<TailPairs<G>, FT, G, NT>(m, a.tail_src, s_done, s_piv);
-            __syncthreads();
-        }
+        if (m > 0) tail_by_waves<TailPairs<G>, FT, G, NT>(m, a.tail_src, s_done, s_piv);
+        __syncthreads();  // (without a tail too: s_piv of the walk, set after its last level's barrier)
         tmark(2);
         // zero / non-finite pivot: klu_factor failure on the first factorisation of a fresh solver
         // (KLUSolver.cpp:38-44), klu_refactor failure afterwards (:50-57)

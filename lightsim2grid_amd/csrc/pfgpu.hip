@@ -802,8 +802,8 @@ __global__ void __launch_bounds__(NT) k_nr(const KArgs a) {
                 dense_tail_lds<FT, G, NT>(Xl, a.m, g, s, act, bad_t);
                 if (bad_t && s == 0) s_piv[g] = 1;
             }
-            __syncthreads();
         }
+        __syncthreads();  // (without a tail too: s_piv of the walk, set after its last level's barrier)
         tmark(2);
         // zero / non-finite pivot: klu_factor failure on the first factorisation of a fresh
         // solver (KLUSolver.cpp:38-44), klu_refactor failure afterwards (:50-57)
