@@ -755,8 +755,9 @@ __global__ void __launch_bounds__(NT, 4) k_nr_block(const BArgs a) {
                 c[0] = c[1] = c[2] = c[3] = (FT)0;
                 return (wu & kBlkLevel) != 0;
             });
-            if (bad) s_piv[g] = 1;
-            if (grow) s_grow[g] = 1;
+            // (lanes of an instance that is done walk along over what its last iteration left)
+            if (act && bad) s_piv[g] = 1;
+            if (act && grow) s_grow[g] = 1;
         }
         tmark(1);
         // ---- dense tail ---------------------------------------------------------------------------

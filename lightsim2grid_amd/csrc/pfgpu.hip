@@ -789,8 +789,9 @@ __global__ void __launch_bounds__(NT) k_nr(const KArgs a) {
                 process(C, Cv, B, Bv);
             }
             }
-            if (bad) s_piv[g] = 1;
-            if (grow) s_grow[g] = 1;
+            // (lanes of an instance that is done walk along over what its last iteration left)
+            if (act && bad) s_piv[g] = 1;
+            if (act && grow) s_grow[g] = 1;
         }
         tmark(1);
         // ---- dense tail: the m x m tile of every instance ---------------------------------
