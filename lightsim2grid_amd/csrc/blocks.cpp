@@ -472,6 +472,13 @@ BlockPlan by_life(BlockPlan P) {
     return P;
 }
 
+int lds_pairs(const BlockPlan& P, size_t room) {
+    if (room >= (size_t)P.npairs) return P.npairs;
+    int q = (int)room;
+    while (q > 0 && P.second[q]) --q;
+    return q;
+}
+
 // ---------------------------------------------------------------------------
 // Unit streams
 // ---------------------------------------------------------------------------

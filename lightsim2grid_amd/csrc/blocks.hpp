@@ -91,6 +91,10 @@ BlockPlan build_block_plan(const YbusPattern& Y, const JPattern& J, const std::v
 // a plan in order kByUse, in order kByLife
 BlockPlan by_life(BlockPlan P);
 
+// Pairs in LDS of a launch with room for `room` of an instance's: all of them, or as many as end between two
+// blocks.
+int lds_pairs(const BlockPlan& P, size_t room);
+
 // Unit streams of the block plan for one launch shape: G interleaved instances, `waves` waves per
 // workgroup, values of fsize bytes, the first nlds pairs in LDS. Each wave has a stream of its own of
 // units of 64 lanes x 4 ints, one product per lane and unit, in level order:

@@ -2081,8 +2081,7 @@ BlockChoice block_shape(const pfgpu_ctx* ctx, const pfgpu_grid::Block& b, int G,
     c.NT = values(c.G) > avail(c.G, 1024) / 2 ? 1024 : 256;
     if (NT_req == 256 || NT_req == 1024) c.NT = NT_req;
     const size_t room = avail(c.G, c.NT), pair = (size_t)2 * c.G * fsize;
-    c.nlds = (int)std::min<size_t>((size_t)P.npairs, room / pair);
-    while (c.nlds < P.npairs && c.nlds > 0 && P.second[c.nlds]) --c.nlds;  // between two blocks
+    c.nlds = pfgpu::lds_pairs(P, room / pair);
     if ((size_t)c.nlds < fixed_pairs) throw ApiError(PFGPU_E_INVALID, "the grid's dense tail does not fit in LDS");
     c.nspill = P.npairs - c.nlds;
     c.lean = c.nspill == 0;
