@@ -2134,15 +2134,36 @@ pfgpu_grid::Block::Lanes& block_lanes(pfgpu_grid::Block& b, const BlockChoice& c
 
 std::unique_ptr<pfgpu_grid::Block> upload_blocks(const pfgpu_grid* g, pfgpu::BlockPlan plan);
 
-// One NR launch on the block plan; as launch_pass otherwise.
+// One NR launch on the block plan; as launch_pass otherwise. G_req -1: the launch with the shortest time for one
+// instance, on as many workgroups as the context's budget holds, the least of them one, which takes all in turn.
 void launch_block(pfgpu_ctx* ctx, pfgpu_grid* gr, const SolveArgs& q, int precision, int G_req, int NT_req, int nunits,
                   const int* imap, const AuxLayout& AL, bool fresh, pfgpu_stats* st, const FixedScratch* fx) {
     const int fsize = precision == PFGPU_FP64 ? 8 : 4;
+    const bool shortest = G_req == -1;
+    if (shortest) {
+        G_req = 1;
+        NT_req = 1024;
+    }
     BlockChoice c = choose_block(ctx, *gr->blk, nunits, fsize, G_req, NT_req);
     auto rows_of = [&](const BlockChoice& x) {  // workspace of a workgroup
         return (size_t)x.G * gr->P.n * 16 + (size_t)x.nspill * 2 * x.G * fsize;
     };
-    if (fx && G_req == 0 && c.G > 1 && rows_of(c) + 1024 > fx->ws_bytes)
+    const int nrow = (int)gr->blk->P.row_len.size(), nent = (int)gr->blk->P.jd_pos.size();
+    const bool gather = q.Yx_stride == 0;
+    const size_t o_yrow = align_up((size_t)std::max(nent, 1) * 16);
+    const size_t gather_bytes = gather ? o_yrow + align_up((size_t)std::max(nrow, 1) * 16) : 0;
+    // workgroups whose rows fit `bytes` of workspace (4 * 256 bytes covers the roundings)
+    auto held = [&](const BlockChoice& x, size_t bytes) -> long long {
+        const size_t per_block = rows_of(x), fixed = gather_bytes + (q.Jx_last ? align_up((size_t)gr->P.n * 16) : 0) + 1024;
+        return bytes <= fixed ? 0 : per_block ? (long long)((bytes - fixed) / per_block) : LLONG_MAX;
+    };
+    auto wanted = [&](const BlockChoice& x) {
+        const void* fn = pfgpu_block::kernel(fsize, x.G, x.NT, x.lean);
+        return std::min<long long>(((long long)nunits + x.G - 1) / x.G, resident_blocks_cached(ctx, fn, x.NT, x.lds));
+    };
+    // several instances per workgroup of a plan that spills, not asked for: one where their workspace does not fit
+    // (10 000 buses in FP64: 1.5 GB with four, 0.35 GB with one)
+    if (G_req == 0 && c.G > 1 && (fx ? held(c, fx->ws_bytes) < 1 : !c.lean && held(c, ctx->budget) < wanted(c)))
         c = block_shape(ctx, *gr->blk, 1, fsize, NT_req);
     pfgpu_grid::Block* use = gr->blk.get();
     if (c.lean && c.v_off < 0) {  // V does not fit beside the values: over some of them?
@@ -2164,17 +2185,12 @@ void launch_block(pfgpu_ctx* ctx, pfgpu_grid* gr, const SolveArgs& q, int precis
     if (static_lds_of(fn) != 0)  // units carry LDS addresses: the values must start at address 0
         throw ApiError(PFGPU_E_INTERNAL, "the NR kernel has static LDS: unit offsets would not be LDS addresses");
     int nres = (int)std::min<long long>(ngroups, resident_blocks_of(ctx, fn, c.NT, c.lds));
-    const int nrow = (int)P.row_len.size(), nent = (int)P.jd_pos.size();
-    const bool gather = q.Yx_stride == 0;
-    const size_t o_yrow = align_up((size_t)std::max(nent, 1) * 16);
-    const size_t gather_bytes = gather ? o_yrow + align_up((size_t)std::max(nrow, 1) * 16) : 0;
     if (fx) {
-        // workgroups whose rows fit the fixed workspace (4 * 256 bytes covers the roundings)
-        const size_t per_block = rows_of(c);
-        const size_t room = fx->ws_bytes > gather_bytes + 1024 ? fx->ws_bytes - gather_bytes - 1024 : 0;
-        const long long cap = per_block ? (long long)(room / per_block) : nres;
+        const long long cap = held(c, fx->ws_bytes);
         if (cap < 1) throw ApiError(PFGPU_E_BUDGET, "the grid's per-workgroup rows do not fit the fixed scratch");
         nres = (int)std::min<long long>(nres, cap);
+    } else if (shortest) {
+        nres = (int)std::min<long long>(nres, std::max(1LL, held(c, ctx->budget)));
     }
     const long long slots = (long long)nres * c.G;
     size_t off = 0;
@@ -2245,7 +2261,7 @@ void launch_pass(pfgpu_ctx* ctx, pfgpu_grid* gr, const SolveArgs& q, int precisi
         // 2000 buses 0.51 against 2.3 wide, 5000 1.3 (0.9) against 3.4, 10 000 4.0 (2.8) against 8.2 (7.7),
         // 20 000 9.8 (7.3) against 25 (22), 40 000 24 (18) against 51 (45).
         if (gr->blk) {
-            launch_block(ctx, gr, q, precision, 1, 1024, nunits, imap, AL, fresh, st, fx);
+            launch_block(ctx, gr, q, precision, -1, 0, nunits, imap, AL, fresh, st, fx);
             if (st) st->instances_per_wg = -1;
         } else {
             launch_wide(ctx, gr, q, precision, nunits, imap, AL, fresh, st);
