@@ -51,37 +51,10 @@ __device__ __forceinline__ double inst_reduce(double v, lds_dbl* part) {
     return r;
 }
 
-// J value at the current V / Ibus (dS_dVa / dS_dVm, BaseNRAlgo.tpp:202-260) of a J entry
-// with selector sel (0/1: Re/Im dS_dVa, 2/3: Re/Im dS_dVm, 4: constant cv) built on the
-// Ybus entry y = Y(r, c); diag says r == c.
-__device__ __forceinline__ double jvalue_of(int sel, bool diag, c64 y, c64 vr, c64 vc, c64 ib, double cv) {
-    if (sel == 4) return cv;
-    if (sel >= 2) {
-        const double ic = 1.0 / sqrt(vc.re * vc.re + vc.im * vc.im);
-        c64 d = cmul(cconj(cmul(y, {vc.re * ic, vc.im * ic})), vr);
-        if (diag) {
-            const double ir = 1.0 / sqrt(vr.re * vr.re + vr.im * vr.im);
-            d = cadd(d, cmul(cconj(ib), {vr.re * ir, vr.im * ir}));
-        }
-        return sel == 2 ? d.re : d.im;
-    }
-    c64 t = cmul(y, vc);
-    if (diag) t = csub(t, ib);
-    const c64 d = cmul(cconj({-t.re, -t.im}), {-vr.im, vr.re});  // * (j V_r)
-    return sel == 0 ? d.re : d.im;
-}
-
-// Orders LDS accesses between the lanes of one wave (they run in lockstep; the
-// fence makes the compiler wait for outstanding LDS operations and not reorder).
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-    __builtin_amdgcn_wave_barrier();
-}
-
 __device__ __forceinline__ double inf_if_nonfinite(double a) { return (a <= 1.7976931348623157e308) ? a : INFINITY; }
 
-// Polar <-> rectangular conversions of one lane's buses (b0, b0 + step, ...).
-// Kept out of line: inlined FP64 atan2 / sincos raise the NR kernel's register
+// Polar form of one lane's buses (b0, b0 + step, ...).
+// Kept out of line: an inlined FP64 atan2 raises the NR kernel's register
 // count past 128 VGPRs, which at 1024 lanes per workgroup means scratch spills
 // in the factor loop.
 // Va = arg(V), Vm = |V| (BaseNRAlgo.tpp:77-79, BaseNRSingleSlackAlgo.tpp:131-132)
@@ -95,22 +68,6 @@ __device__ __noinline__ void polar_of(VP V, int vs, double* __restrict__ Va, dou
         Vm[b] = sqrt(vr * vr + vi * vi);
     }
 }
-// V = Vm * exp(j Va) (BaseNRAlgo.tpp:150-151); returns min Vm over the lane's buses
-template <typename VP>
-__device__ __noinline__ double rect_of(VP V, int vs, const double* __restrict__ Va, const double* __restrict__ Vm,
-                                       int b0, int n, int step) {
-    double vmin = INFINITY;
-    for (int b = b0; b < n; b += step) {
-        double sn, cs;
-        sincos(Va[b], &sn, &cs);
-        const double m = Vm[b];
-        V[2 * b * vs] = m * cs;
-        V[2 * b * vs + 1] = m * sn;
-        vmin = fmin(vmin, m);
-    }
-    return vmin;
-}
-
 // One bus of the voltage update (BaseNRAlgo.tpp:138-151): Va and Vm (taken from V first in
 // the single-slack form, BaseNRSingleSlackAlgo.tpp:131-132) minus the Newton step, then
 // V = Vm exp(j Va); returns Vm.
