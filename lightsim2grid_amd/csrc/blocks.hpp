@@ -3,7 +3,7 @@
 //
 // One block product replaces up to 8 scalar ones, and the dependency chains count buses instead of
 // unknowns: on the 2000-bus grid 28 474 products in 33 levels where the scalar schedule has 136 790
-// in 53 (10 000 buses: 185 444 in 51 against 834 922 in 82). The pattern is the exact one of the
+// in 53 (10 000 buses: 214 561 in 71 against 834 922 in 82). The pattern is the exact one of the
 // static elimination (L and U apart), so the reference slack's row takes no part where it is zero.
 //
 // Values are stored as pairs (2 consecutive numbers of one instance). A factor block (i, k) of L has
@@ -38,8 +38,9 @@ constexpr int kBlkWide = (int)(1u << 31);          // the block of U has two col
                                                    // wave lies outside LDS (factor)
 
 // Unknowns of the dense tail at most: a wave factors it in registers, a column to a register and a row to
-// a lane (nr_block_kernel.hpp), which at 1024 lanes leaves room for 48 columns of FP64. (The 10 000-bus grid's top chain has 88 unknowns: the
-// 40 below the tail take 20 levels more, as long as the 40 took in a tail of 16 waves.)
+// a lane (nr_block_kernel.hpp), which at 1024 lanes leaves room for 48 columns of FP64. (The 10 000-bus grid's
+// top chain has 88 unknowns: the 40 below the tail take 20 levels more, as long as the 40 took in a tail of 16
+// waves.)
 constexpr int kMaxTail = 48;
 
 struct BlockPlan {

@@ -2041,9 +2041,12 @@ BlockChoice choose_block(const pfgpu_ctx* ctx, const pfgpu_grid::Block& b, int n
     const long long ncu = std::max(1, ctx->n_cu);
     if (ninst <= ncu) return best;
     // FP64 values of five times the LDS and more: most operands are read from memory, where four instances side
-    // by side make whole cache lines. Of the 10 000-bus grid a round of G = 1, 2, 4 takes 4.4, 7.1, 11.4 ms
-    // (G = 1 and 4: 9692 outages 166, 108 ms; 2000 34.6, 23.4; 600 11.2, 13.1); of the 3000-bus grid, 2.6 times the
-    // LDS, 0.75, 1.6, 2.7. In FP32 (10 000 buses) 2.2, 5.4, 9.1.
+    // by side make whole cache lines. Kernel time in ms with G = 1 and 4, 2000 outages (1100; 600) of grids of
+    // 2.5 times the LDS (3000 buses): 4.9, 5.2 (2.9, 3.3; 1.7, 2.5); of 4.2 (5000): 10.6, 9.8 (6.3, 6.3; 3.6, 5.0);
+    // of 5 (6000): 13.0, 11.8 (7.7, 7.5; 4.4, 6.0); of 5.9 (7000): 18.1, 14.5 (10.5, 9.2; 6.1, 7.3); of 8.2
+    // (10 000): 35.0, 31.1 (19.8, 24.6: a second round for 19 groups; 12.8, 21.4). G = 2 lies between or above
+    // but for 2000 outages of 10 000 buses (29.0). FP32 values stay at G = 1: nothing but the autotuner looks
+    // further there, which finds G = 8 on 9692 outages of 10 000 buses (76 against 84 ms).
     if (fsize == 8 && (size_t)b.P.npairs * 16 >= 5 * (size_t)ctx->lds_max) {
         const double one = (double)ninst / (double)ncu;
         if (std::max(one / 4, 1.0) * 2.6 < one) {
