@@ -78,11 +78,12 @@ int ServeLoop::add_grid(const CscC& Y, const CplxVect& Sbus, const CplxVect& V0,
              "pfgpu_grid_load");
     pfgpu_grid_info info{};
     check_rc(pfgpu_grid_get_info(g->grid, &info), "pfgpu_grid_get_info");
-    // per-instance device bytes of a launch: Ybus values (contingencies), Va/Vm/Ibus, spilled
-    // value slots (upper bound), Sbus / V in / V out, iterations and status
-    // transient device bytes one instance of a launch may take in the engine (at most): Va, Vm and
-    // Ibus rows, FP64 spilled value slots, flags and fallback list
-    g->bytes_per_inst = (size_t)n * 32 + (size_t)info.n_slots * 8 + 64;
+    // transient device bytes one instance of a launch may take in the engine (at most): Va and Vm rows, FP64
+    // values outside LDS, flags and fallback list. One instance to a workgroup leaves it all of a compute unit's
+    // LDS, 128 KB and more of values; an eighth is taken off small plans, whose values all lie there. (The scalar
+    // kernel of a re-pivoted plan has Ibus rows too, and fewer slots.)
+    const size_t values = (size_t)info.n_slots * 8;
+    g->bytes_per_inst = (size_t)n * 16 + values - std::min(values / 8, (size_t)128 << 10) + 64;
     auto alloc = [&](double** p, size_t bytes) {
         void* q = nullptr;
         check_rc(pfgpu_dev_alloc(g->ctx, bytes, &q), "pfgpu_dev_alloc");
