@@ -2158,16 +2158,20 @@ void launch_block(pfgpu_ctx* ctx, pfgpu_grid* gr, const SolveArgs& q, int precis
     // workgroups whose rows fit `bytes` of workspace (4 * 256 bytes covers the roundings)
     auto held = [&](const BlockChoice& x, size_t bytes) -> long long {
         const size_t per_block = rows_of(x), fixed = gather_bytes + (q.Jx_last ? align_up((size_t)gr->P.n * 16) : 0) + 1024;
-        return bytes <= fixed ? 0 : per_block ? (long long)((bytes - fixed) / per_block) : LLONG_MAX;
+        return bytes <= fixed ? 0 : per_block ? (long long)((bytes - fixed) / per_block) : INT_MAX;
     };
     auto wanted = [&](const BlockChoice& x) {
         const void* fn = pfgpu_block::kernel(fsize, x.G, x.NT, x.lean);
         return std::min<long long>(((long long)nunits + x.G - 1) / x.G, resident_blocks_cached(ctx, fn, x.NT, x.lds));
     };
-    // several instances per workgroup of a plan that spills, not asked for: one where their workspace does not fit
-    // (10 000 buses in FP64: 1.5 GB with four, 0.35 GB with one)
-    if (G_req == 0 && c.G > 1 && (fx ? held(c, fx->ws_bytes) < 1 : !c.lean && held(c, ctx->budget) < wanted(c)))
-        c = block_shape(ctx, *gr->blk, 1, fsize, NT_req);
+    // Fewer instances per workgroup where the workspace of these does not fit: one if the number was not asked for,
+    // else half as many. (The scalar plan's tail held 10 000 buses to two per workgroup in FP64 and four in FP32,
+    // 0.71 and 0.87 GB; four and eight take 1.49 and 1.68, one 0.34 and 0.17.) Three quarters of the workgroups are
+    // enough: pairs padded to blocks take up to 15 % more than the scalar plan's slots did.
+    auto fits = [&](const BlockChoice& x) {
+        return fx ? held(x, fx->ws_bytes) >= 1 : 4 * held(x, ctx->budget) >= 3 * wanted(x);
+    };
+    while (c.G > 1 && (!fx || G_req == 0) && !fits(c)) c = block_shape(ctx, *gr->blk, G_req == 0 ? 1 : c.G / 2, fsize, NT_req);
     pfgpu_grid::Block* use = gr->blk.get();
     if (c.lean && c.v_off < 0) {  // V does not fit beside the values: over some of them?
         if (!gr->blk_life && !fx) gr->blk_life = upload_blocks(gr, pfgpu::by_life(gr->blk->P));
@@ -2192,8 +2196,8 @@ void launch_block(pfgpu_ctx* ctx, pfgpu_grid* gr, const SolveArgs& q, int precis
         const long long cap = held(c, fx->ws_bytes);
         if (cap < 1) throw ApiError(PFGPU_E_BUDGET, "the grid's per-workgroup rows do not fit the fixed scratch");
         nres = (int)std::min<long long>(nres, cap);
-    } else if (shortest) {
-        nres = (int)std::min<long long>(nres, std::max(1LL, held(c, ctx->budget)));
+    } else if (const long long cap = held(c, ctx->budget); shortest || 4 * cap >= 3LL * nres) {
+        nres = (int)std::min<long long>(nres, std::max(1LL, cap));
     }
     const long long slots = (long long)nres * c.G;
     size_t off = 0;

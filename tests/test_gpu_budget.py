@@ -67,3 +67,48 @@ def test_large_fp64_batch_in_a_smaller_budget(gpu_ctx):
     assert np.array_equal(r4["status"], r1["status"]) and np.array_equal(r4["iters"], r1["iters"])
     ok = r1["status"] == 0
     assert np.max(np.abs(r4["V"][ok] - r1["V"][ok])) <= 1e-9
+
+
+@pytest.mark.parametrize("name,rows,prec,G,budget", [("case10000_synth", 1100, 0, 8, 720e6), ("case10000_synth", 1100, 0, 1, 337e6),
+                                                     ("case2000_synth", 600, 0, 1, 37.5e6), ("case118_synth", 9000, 0, 32, 95e6)])
+def test_shapes_asked_for_in_a_budget_of_the_scalar_plans(gpu_ctx, name, rows, prec, G, budget):
+    """What the scalar plan of a grid took for a launch shape is enough for the block plan's, at the most with fewer
+    instances or workgroups side by side."""
+    from lightsim2grid_amd import abi, gridgen
+    _say("small budget, shapes", name, rows, prec, G)
+    g = gridgen.make(name)
+    V = _base(gpu_ctx, g)
+    want = _solve(gpu_ctx, g, V, rows, prec, G)
+    ctx = abi.Context(0, int(budget))
+    got = _solve(ctx, g, V, rows, prec, G)
+    ctx.close()
+    assert np.array_equal(got["status"], want["status"]) and np.array_equal(got["iters"], want["iters"])
+    ok = want["status"] == 0
+    assert np.max(np.abs(got["V"][ok] - want["V"][ok])) <= 1e-9
+    if G in (1, 32):
+        assert got["stats"]["instances_per_wg"] == G and np.array_equal(got["V"], want["V"])
+
+
+def test_autotune_in_a_budget_of_the_scalar_plans(gpu_ctx):
+    from lightsim2grid_amd import abi, gridgen
+    _say("small budget, autotune")
+    g = gridgen.make("case10000_synth")
+    d = g.solver_inputs()
+    V, rows = _base(gpu_ctx, g), 520
+    lines = np.nonzero(~gridgen.bridges(g))[0]
+    deltas = g.ybus_deltas([[int(k)] for k in lines[:rows]])
+    out = []
+    for ctx in (gpu_ctx, abi.Context(0, 720_000_000)):
+        gr = abi.Grid(ctx, d["Ybus"], d["slack_ids"], d["slack_weights"], d["pv"], d["pq"])
+        dev = ctx.to_device
+        a = (dev(gr.ybus_values(d["Ybus"])), 0, dev(np.ascontiguousarray(d["Sbus"])), 0, dev(V), 0,
+             ctx.empty((rows, g.n), np.complex128), rows, ctx.empty(rows, np.int32), ctx.empty(rows, np.int32))
+        dd = tuple(dev(x) for x in deltas)
+        if ctx is not gpu_ctx:
+            gr.autotune_device(*a, precision=0, deltas=dd)
+        gr.solve_device(*a, precision=0, deltas=dd)
+        out.append((a[9].to_host(), a[8].to_host(), a[6].to_host()))
+        gr.close()
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
+    ok = out[0][0] == 0
+    assert np.max(np.abs(out[0][2][ok] - out[1][2][ok])) <= 1e-9
