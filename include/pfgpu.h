@@ -74,7 +74,8 @@ typedef struct pfgpu_grid_info {
     int nnz_ybus;
     int nnz_jac;
     int64_t nnz_lu;     /* diag + L + U entries of the static-pivot factor */
-    int n_slots;        /* per-instance value slots (LU + forward-solve vector) */
+    int n_slots;        /* per-instance value slots (LU + forward-solve vector; of a plan by bus
+                         * blocks two per pair of values, padding included) */
     int n_levels;       /* factor + forward dependency levels */
     int n_back_levels;  /* backward-solve levels */
     int64_t n_pairs;    /* multiply pairs of one refactorisation + forward solve */
@@ -186,13 +187,14 @@ int pfgpu_grid_get_J_pattern(const pfgpu_grid* grid, int* Jp, int* Ji);
  *             initial vector of every instance (V still receives ninst rows)
  *   precision PFGPU_FP64, PFGPU_FP32 or PFGPU_FP32_STRICT (see above)
  *   instances_per_wg  0 = automatic, else G in {1,2,4,8,16,32}; -1 = the launch with the
- *             shortest time for one instance: a workgroup of 1024 lanes each or, on a plan
- *             without a block form (pivots off J's diagonal, more than 2^20 value pairs), the
- *             instances one after the other, each spread over 32 workgroups
- *             (PFGPU_WIDE_BLOCKS) that run the NR phases and each elimination level together,
- *             separated by grid-wide barriers (cooperative launch). Automatic for a single
- *             instance (or a single chain) of a plan with at least 200000 factor pairs;
- *             pfgpu_stats.instances_per_wg is -1 then. Not for DC grids.
+ *             shortest time for one instance: a workgroup of 1024 lanes each, as many side by
+ *             side as the HBM budget holds, or, on a plan without a block form (pivots off J's
+ *             diagonal, more than 2^20 value pairs), the instances one after the other, each
+ *             spread over 32 workgroups (PFGPU_WIDE_BLOCKS) that run the NR phases and each
+ *             elimination level together, separated by grid-wide barriers (cooperative
+ *             launch). Automatic for a single instance (or a single chain) of a plan with at
+ *             least 200000 factor pairs; pfgpu_stats.instances_per_wg is -1 then. Not for DC
+ *             grids.
  *   iters/status      [ninst] outputs: NR iterations (linear solves) and the
  *             ErrorType (0 converged)
  *   Jx_last   optional [nnz_jac] J values of instance 0's last iteration (or NULL)
